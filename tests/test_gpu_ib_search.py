@@ -271,3 +271,41 @@ def test_tangent_projection_fallback_records_invalid_count():  # :1272-1300
     assert search.nearest_marker_index((0, 0, 0)) == 0
     assert search.boundary_point_m((0, 0, 0)) == (0.5, 0.5, 0.5)
     assert search.interior_fluid_point_m((0, 0, 0)) == (0.5, 0.5, 0.625)
+
+
+@pytest.mark.parametrize("sizes", [(0.6,), (0.05,), (0.3, 0.1), (0.001,)])
+@pytest.mark.parametrize("sliver", [1.0, 40.0])
+def test_far_bounds_skip_nothing_that_counts(sizes, sliver):
+    """Far classification below open patches that face up, so that most nodes under them are internal and
+    take the nearest of all triangles: large, small and tiny patches far from most nodes (where the
+    closest-point formula loses digits and nothing may be skipped), two at different heights, slivers
+    (one axis squeezed), every fifth triangle twice (equal distances: the lower index)."""
+    rng = np.random.default_rng(int(1000 * sizes[0]) + int(sliver))
+    xm, nm, tris = [], [], []
+    m = 9
+    for q, size in enumerate(sizes):
+        u, v = np.meshgrid(np.linspace(-0.5, 0.5, m), np.linspace(-0.5, 0.5, m), indexing="ij")
+        h = 0.05 * (u * u + v * v) + 0.002 * rng.normal(size=u.shape)
+        x = np.stack([u.ravel() * size / sliver, v.ravel() * size, h.ravel() * size], -1)
+        at = len(xm) * m * m
+        xm.append((x + (0.3 + 0.3 * q, 0.47, 0.62 + 0.1 * q)).astype(np.float32))
+        nm.append(np.tile(np.array([0, 0, 1], np.float32), (m * m, 1)))
+        for i in range(m - 1):
+            for j in range(m - 1):
+                c = at + i * m + j
+                tris += [(c, c + m, c + m + 1), (c, c + m + 1, c + 1)]
+    xm, nm = np.concatenate(xm), np.concatenate(nm)
+    tris = [t for k, t in enumerate(tris) for _ in range(2 if k % 5 == 0 else 1)]
+    shape = (21, 18, 23)
+    _say(f"ib search: open patches {sizes}, sliver {sliver}, {len(tris)} triangles")
+    search = _search(shape, capacity=len(xm))
+    markers = _markers(xm, nm, tris)
+    rep = search.search_and_classify(markers, search_radius_m=0.03, interior_probe_distance_m=0.02,
+                                     classify_far_internal_nodes=True)
+    want, rep_want = S.search_and_classify(_positions(search), markers.x_gamma_m.to_numpy(),
+                                           markers.n_gamma.to_numpy(), tris, search_radius=0.03,
+                                           interior_probe_distance=0.02,
+                                           sign_tolerance=search._default_sign_tolerance_m(),
+                                           classify_far_internal_nodes=True)
+    _compare(search, want, rep_want, rep)
+    assert rep.internal_node_count > 50
