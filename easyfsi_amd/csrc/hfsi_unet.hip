@@ -28,11 +28,15 @@ void set_error(const std::string& msg);
 
 enum { E1A, E1B, E2A, E2B, B3A, B3B, D2A, D2B, D1A, D1B, NCONV };
 
+static_assert((int)NCONV == kConvLayers, "layer tables");
+
 struct UConv {
   int cin, cout, cin_true;
   size_t w_off, b_off;
   bf16* wf = nullptr;  // forward weights [cout][KP(cin)]
   bf16* wb = nullptr;  // data-gradient weights [cin][KP(cout)] (null for E1A)
+  float* partial = nullptr;  // partial weight and bias gradients of `parts` workgroups per 16 input channels
+  int parts = 0;
 };
 
 static inline int grid1d(long n, int threads = 256) {
@@ -57,8 +61,6 @@ struct hfsi_unet {
   bf16 *g_a1 = nullptr, *g_s1 = nullptr, *g_p1 = nullptr, *g_a2 = nullptr, *g_s2 = nullptr, *g_p2 = nullptr,
        *g_a3 = nullptr, *g_b3 = nullptr, *g_u2 = nullptr, *g_a4 = nullptr, *g_d2 = nullptr, *g_u1 = nullptr,
        *g_a5 = nullptr, *g_d1 = nullptr;
-  float* wpartial = nullptr;
-  float* bpartial = nullptr;
   double* partials = nullptr;
   double* totals = nullptr;
   double* host_totals = nullptr;
@@ -83,22 +85,22 @@ static int ualloc(hfsi_unet* h, T** out, size_t count) {
 // ---- dispatch over the channel pairs of the topology ----------------------
 
 template <int CI, int CO>
-static void conv_fwd_t(const bf16* x, const bf16* w, const float* b, bf16* y, int D, int H, int W, bool relu,
-                       hipStream_t st) {
+static void conv_fwd_t(const bf16* x, const bf16* w, const float* b, const bf16* gate, bf16* y, int D, int H, int W,
+                       bool relu, hipStream_t st) {
   const int blocks = conv_blocks(D, H, W);
   if (relu)
-    hipLaunchKernelGGL((k_conv3_fwd<CI, CO, true>), dim3(blocks), dim3(kConvThreads), 0, st, x, w, b, y, CO, 0, D, H,
-                       W);
+    hipLaunchKernelGGL((k_conv3_fwd<CI, CO, true>), dim3(blocks), dim3(kConvThreads), 0, st, x, w, b, gate, y, CO, 0,
+                       D, H, W);
   else
-    hipLaunchKernelGGL((k_conv3_fwd<CI, CO, false>), dim3(blocks), dim3(kConvThreads), 0, st, x, w, b, y, CO, 0, D,
-                       H, W);
+    hipLaunchKernelGGL((k_conv3_fwd<CI, CO, false>), dim3(blocks), dim3(kConvThreads), 0, st, x, w, b, gate, y, CO, 0,
+                       D, H, W);
 }
 
-static int conv_fwd(int ci, int co, const bf16* x, const bf16* w, const float* b, bf16* y, int D, int H, int W,
-                    bool relu, hipStream_t st) {
+static int conv_fwd(int ci, int co, const bf16* x, const bf16* w, const float* b, const bf16* gate, bf16* y, int D,
+                    int H, int W, bool relu, hipStream_t st) {
 #define HFSI_CONV_CASE(A, B)                                 \
   if (ci == A && co == B) {                                  \
-    conv_fwd_t<A, B>(x, w, b, y, D, H, W, relu, st);         \
+    conv_fwd_t<A, B>(x, w, b, gate, y, D, H, W, relu, st);   \
     return HFSI_OK;                                          \
   }
   HFSI_CONV_CASE(16, 16)
@@ -118,52 +120,45 @@ static int conv_fwd(int ci, int co, const bf16* x, const bf16* w, const float* b
   return HFSI_ERR_ARG;
 }
 
-static int wgrad_chunks(long n, int* chunk) {
-  long nch = (n + 1023) / 1024;
-  if (nch > 64) nch = 64;
-  if (nch < 1) nch = 1;
-  long c = (n + nch - 1) / nch;
-  c = (c + kWgStep - 1) / kWgStep * kWgStep;
-  *chunk = (int)c;
-  return (int)((n + c - 1) / c);
+static size_t wgrad_partial_size(const UConv& L, int D, int H, int W) {
+  return (size_t)(L.cin / 16) * wgrad_parts(conv_tiles(D, H, W), L.cin) * kWgTaps * L.cout * 16;
 }
 
 template <int CI, int CO>
-static void conv_wgrad_t(const bf16* x, const bf16* dy, float* partial, int D, int H, int W, int nch, int chunk,
-                         hipStream_t st) {
-  hipLaunchKernelGGL((k_conv3_wgrad<CI, CO>), dim3(nch, 27), dim3(kConvThreads), 0, st, x, dy, partial, D, H, W,
-                     chunk);
+static void conv_wgrad_t(const bf16* x, const bf16* dy, float* partial, int D, int H, int W, hipStream_t st) {
+  hipLaunchKernelGGL((k_conv3_wgrad<CI, CO>), dim3(wgrad_parts(conv_tiles(D, H, W), CI), CI / 16), dim3(kConvThreads),
+                     0, st, x, dy, partial, D, H, W);
 }
 
-static int conv_wgrad(hfsi_unet* h, const UConv& L, const bf16* x, const bf16* dy, int D, int H, int W,
-                      hipStream_t st) {
-  const long n = (long)D * H * W;
-  int chunk = 0;
-  const int nch = wgrad_chunks(n, &chunk);
-  const int ci = L.cin, co = L.cout;
-  bool ok = true;
-  if (ci == 16 && co == 16) conv_wgrad_t<16, 16>(x, dy, h->wpartial, D, H, W, nch, chunk, st);
-  else if (ci == 16 && co == 32) conv_wgrad_t<16, 32>(x, dy, h->wpartial, D, H, W, nch, chunk, st);
-  else if (ci == 32 && co == 32) conv_wgrad_t<32, 32>(x, dy, h->wpartial, D, H, W, nch, chunk, st);
-  else if (ci == 32 && co == 64) conv_wgrad_t<32, 64>(x, dy, h->wpartial, D, H, W, nch, chunk, st);
-  else if (ci == 64 && co == 64) conv_wgrad_t<64, 64>(x, dy, h->wpartial, D, H, W, nch, chunk, st);
-  else if (ci == 96 && co == 32) conv_wgrad_t<96, 32>(x, dy, h->wpartial, D, H, W, nch, chunk, st);
-  else if (ci == 48 && co == 16) conv_wgrad_t<48, 16>(x, dy, h->wpartial, D, H, W, nch, chunk, st);
-  else ok = false;
-  if (!ok) {
-    set_error("hfsi_unet: unsupported weight-gradient shape");
-    return HFSI_ERR_ARG;
+// The layer's partial weight and bias gradients (summed for all layers by k_grad_reduce).
+static int conv_wgrad(const UConv& L, const bf16* x, const bf16* dy, int D, int H, int W, hipStream_t st) {
+#define HFSI_WGRAD_CASE(A, B)                              \
+  if (L.cin == A && L.cout == B) {                         \
+    conv_wgrad_t<A, B>(x, dy, L.partial, D, H, W, st);     \
+    return HFSI_OK;                                        \
   }
-  hipLaunchKernelGGL(k_wgrad_reduce, dim3(grid1d(27L * ci * co)), dim3(256), 0, st, (const float*)h->wpartial, nch,
-                     ci, co, h->grads + L.w_off);
-  // bias gradient
-  const int nb = grid1d(n / (256 / co) + 1);
-  if (co == 16) hipLaunchKernelGGL((k_bias_grad<16>), dim3(nb), dim3(256), 0, st, dy, n, h->bpartial);
-  else if (co == 32) hipLaunchKernelGGL((k_bias_grad<32>), dim3(nb), dim3(256), 0, st, dy, n, h->bpartial);
-  else hipLaunchKernelGGL((k_bias_grad<64>), dim3(nb), dim3(256), 0, st, dy, n, h->bpartial);
-  hipLaunchKernelGGL(k_bias_reduce, dim3(1), dim3(64), 0, st, (const float*)h->bpartial, nb, co,
-                     h->grads + L.b_off);
-  return HFSI_OK;
+  HFSI_WGRAD_CASE(16, 16)
+  HFSI_WGRAD_CASE(16, 32)
+  HFSI_WGRAD_CASE(32, 32)
+  HFSI_WGRAD_CASE(32, 64)
+  HFSI_WGRAD_CASE(64, 64)
+  HFSI_WGRAD_CASE(96, 32)
+  HFSI_WGRAD_CASE(48, 16)
+#undef HFSI_WGRAD_CASE
+  set_error("hfsi_unet: unsupported weight-gradient shape");
+  return HFSI_ERR_ARG;
+}
+
+// The layers of a pass over all of them, `work(l)` workgroups each; returns the total.
+template <typename F>
+static int conv_layers(const hfsi_unet* h, ConvLayers& tab, F work) {
+  int first = 0;
+  for (int l = 0; l < NCONV; ++l) {
+    const UConv& L = h->conv[l];
+    tab.l[l] = {L.cin, L.cout, L.parts, first, L.partial, L.w_off, L.b_off, L.wf, L.wb};
+    first += work(L);
+  }
+  return first;
 }
 
 // Output-layer gradient accumulation from the combined sums {sum dy u[c], sum dy}.
@@ -180,17 +175,13 @@ struct FinLoss {
   __device__ void operator()(const double*) const {}
 };
 
-static void relu_bwd(bf16* g, const bf16* y, long n, hipStream_t st) {
-  hipLaunchKernelGGL(k_relu_bwd, dim3(grid1d(n)), dim3(256), 0, st, g, y, n);
-}
-
 static int refresh_weights(hfsi_unet* h, hipStream_t st) {
-  for (int l = 0; l < NCONV; ++l) {
-    const UConv& L = h->conv[l];
-    const long n = (long)L.cout * conv_kp(L.cin) + (L.wb ? (long)L.cin * conv_kp(L.cout) : 0);
-    hipLaunchKernelGGL(k_conv_weights, dim3(grid1d(n)), dim3(256), 0, st, (const float*)h->params + L.w_off, L.cin,
-                       L.cout, L.wf, L.wb);
-  }
+  ConvLayers tab;
+  const int blocks = conv_layers(h, tab, [](const UConv& L) {
+    const int n = L.cout * conv_kp(L.cin) + (L.wb ? L.cin * conv_kp(L.cout) : 0);
+    return (n + kWeightsPerBlock - 1) / kWeightsPerBlock;
+  });
+  hipLaunchKernelGGL(k_conv_weights, dim3(blocks), dim3(256), 0, st, tab, (const float*)h->params);
   if (hipGetLastError() != hipSuccess) {
     set_error("hfsi_unet: weight conversion launch failed");
     return HFSI_ERR_HIP;
@@ -284,8 +275,12 @@ int hfsi_unet_create(hfsi_unet** out, int32_t nx, int32_t ny, int32_t nz, int32_
     rc |= ualloc(h, &h->g_u1, n1 * 48);
     rc |= ualloc(h, &h->g_a5, n1 * 16);
     rc |= ualloc(h, &h->g_d1, n1 * 16);
-    rc |= ualloc(h, &h->wpartial, (size_t)64 * 27 * 96 * 32);
-    rc |= ualloc(h, &h->bpartial, (size_t)8192 * 64);
+    for (int l = 0; l < NCONV && rc == HFSI_OK; ++l) {
+      UConv& L = h->conv[l];
+      const int s = l == E2A || l == E2B || l == D2A || l == D2B ? 2 : l == B3A || l == B3B ? 4 : 1;
+      L.parts = wgrad_parts(conv_tiles(nx / s, ny / s, nz / s), L.cin);
+      rc |= ualloc(h, &L.partial, wgrad_partial_size(L, nx / s, ny / s, nz / s));
+    }
   }
   if (rc == HFSI_OK && hipHostMalloc((void**)&h->host_totals, 64 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
     set_error("hfsi_unet_create: hipHostMalloc failed");
@@ -393,20 +388,20 @@ int hfsi_unet_forward(hfsi_unet* h, const float* in5, float* out, void* stream) 
   auto b = [&](int l) { return P + h->conv[l].b_off; };
   hipLaunchKernelGGL(k_unet_input, dim3(grid1d(h->n1)), dim3(256), 0, st, in5, h->x0, h->n1);
   int rc = HFSI_OK;
-  rc |= conv_fwd(16, 16, h->x0, h->conv[E1A].wf, b(E1A), h->a1, D, H, W, true, st);
-  rc |= conv_fwd(16, 16, h->a1, h->conv[E1B].wf, b(E1B), h->s1, D, H, W, true, st);
-  hipLaunchKernelGGL(k_pool2_fwd, dim3(grid1d(h->n2 * 16)), dim3(256), 0, st, h->s1, h->p1, D, H, W, 16);
-  rc |= conv_fwd(16, 32, h->p1, h->conv[E2A].wf, b(E2A), h->a2, D2, H2, W2, true, st);
-  rc |= conv_fwd(32, 32, h->a2, h->conv[E2B].wf, b(E2B), h->s2, D2, H2, W2, true, st);
-  hipLaunchKernelGGL(k_pool2_fwd, dim3(grid1d(h->n3 * 32)), dim3(256), 0, st, h->s2, h->p2, D2, H2, W2, 32);
-  rc |= conv_fwd(32, 64, h->p2, h->conv[B3A].wf, b(B3A), h->a3, D3, H3, W3, true, st);
-  rc |= conv_fwd(64, 64, h->a3, h->conv[B3B].wf, b(B3B), h->b3, D3, H3, W3, true, st);
+  rc |= conv_fwd(16, 16, h->x0, h->conv[E1A].wf, b(E1A), nullptr, h->a1, D, H, W, true, st);
+  rc |= conv_fwd(16, 16, h->a1, h->conv[E1B].wf, b(E1B), nullptr, h->s1, D, H, W, true, st);
+  hipLaunchKernelGGL(k_pool2_fwd, dim3(grid1d(h->n2 * 2)), dim3(256), 0, st, h->s1, h->p1, D, H, W, 16);
+  rc |= conv_fwd(16, 32, h->p1, h->conv[E2A].wf, b(E2A), nullptr, h->a2, D2, H2, W2, true, st);
+  rc |= conv_fwd(32, 32, h->a2, h->conv[E2B].wf, b(E2B), nullptr, h->s2, D2, H2, W2, true, st);
+  hipLaunchKernelGGL(k_pool2_fwd, dim3(grid1d(h->n3 * 4)), dim3(256), 0, st, h->s2, h->p2, D2, H2, W2, 32);
+  rc |= conv_fwd(32, 64, h->p2, h->conv[B3A].wf, b(B3A), nullptr, h->a3, D3, H3, W3, true, st);
+  rc |= conv_fwd(64, 64, h->a3, h->conv[B3B].wf, b(B3B), nullptr, h->b3, D3, H3, W3, true, st);
   hipLaunchKernelGGL(k_upcat_fwd, dim3(grid1d(h->n2 * 12)), dim3(256), 0, st, h->b3, h->s2, h->u2, D2, H2, W2, 64, 32);
-  rc |= conv_fwd(96, 32, h->u2, h->conv[D2A].wf, b(D2A), h->a4, D2, H2, W2, true, st);
-  rc |= conv_fwd(32, 32, h->a4, h->conv[D2B].wf, b(D2B), h->d2, D2, H2, W2, true, st);
+  rc |= conv_fwd(96, 32, h->u2, h->conv[D2A].wf, b(D2A), nullptr, h->a4, D2, H2, W2, true, st);
+  rc |= conv_fwd(32, 32, h->a4, h->conv[D2B].wf, b(D2B), nullptr, h->d2, D2, H2, W2, true, st);
   hipLaunchKernelGGL(k_upcat_fwd, dim3(grid1d(h->n1 * 6)), dim3(256), 0, st, h->d2, h->s1, h->u1, D, H, W, 32, 16);
-  rc |= conv_fwd(48, 16, h->u1, h->conv[D1A].wf, b(D1A), h->a5, D, H, W, true, st);
-  rc |= conv_fwd(16, 16, h->a5, h->conv[D1B].wf, b(D1B), h->d1, D, H, W, true, st);
+  rc |= conv_fwd(48, 16, h->u1, h->conv[D1A].wf, b(D1A), nullptr, h->a5, D, H, W, true, st);
+  rc |= conv_fwd(16, 16, h->a5, h->conv[D1B].wf, b(D1B), nullptr, h->d1, D, H, W, true, st);
   hipLaunchKernelGGL((k_out_fwd<16>), dim3(grid1d(h->n1)), dim3(256), 0, st, h->d1, P + h->w_out_off,
                      P + h->b_out_off, out, h->n1);
   if (rc != HFSI_OK) return rc;
@@ -433,50 +428,47 @@ int hfsi_unet_backward(hfsi_unet* h, const float* dout, void* stream) {
                        (const double*)h->partials, (uint32_t)nb, h->totals,
                        FinOut{h->grads + h->w_out_off, h->grads + h->b_out_off}, (uint64_t)0);
   }
-  HFSI_CHECK(hipMemsetAsync(h->g_s1, 0, n1 * 16 * sizeof(bf16), st));
-  HFSI_CHECK(hipMemsetAsync(h->g_s2, 0, n2 * 32 * sizeof(bf16), st));
+  // Every gradient that is written here has its ReLU applied where it is produced (gates), but those of
+  // the concatenations and pooled tensors, which have none.
+  auto dgrad = [&](int l, const bf16* dy, const bf16* gate, bf16* dx, int d, int hh, int w) {
+    return conv_fwd(h->conv[l].cout, h->conv[l].cin, dy, h->conv[l].wb, nullptr, gate, dx, d, hh, w, false, st);
+  };
   // level 1 decoder
-  relu_bwd(h->g_d1, h->d1, n1 * 16, st);
-  rc |= conv_wgrad(h, h->conv[D1B], h->a5, h->g_d1, D, H, W, st);
-  rc |= conv_fwd(16, 16, h->g_d1, h->conv[D1B].wb, nullptr, h->g_a5, D, H, W, false, st);
-  relu_bwd(h->g_a5, h->a5, n1 * 16, st);
-  rc |= conv_wgrad(h, h->conv[D1A], h->u1, h->g_a5, D, H, W, st);
-  rc |= conv_fwd(16, 48, h->g_a5, h->conv[D1A].wb, nullptr, h->g_u1, D, H, W, false, st);
-  hipLaunchKernelGGL(k_upcat_bwd_coarse, dim3(grid1d(n2 * 32)), dim3(256), 0, st, h->g_u1, h->g_d2, D, H, W, 32, 16);
-  hipLaunchKernelGGL(k_upcat_bwd_skip, dim3(grid1d(n1 * 16)), dim3(256), 0, st, h->g_u1, h->g_s1, n1, 32, 16);
+  rc |= conv_wgrad(h->conv[D1B], h->a5, h->g_d1, D, H, W, st);
+  rc |= dgrad(D1B, h->g_d1, h->a5, h->g_a5, D, H, W);
+  rc |= conv_wgrad(h->conv[D1A], h->u1, h->g_a5, D, H, W, st);
+  rc |= dgrad(D1A, h->g_a5, nullptr, h->g_u1, D, H, W);
+  hipLaunchKernelGGL(k_upcat_bwd_coarse, dim3(grid1d(n2 * 4)), dim3(256), 0, st, h->g_u1, h->d2, h->g_d2, D, H, W, 32,
+                     16);
   // level 2 decoder
-  relu_bwd(h->g_d2, h->d2, n2 * 32, st);
-  rc |= conv_wgrad(h, h->conv[D2B], h->a4, h->g_d2, D2, H2, W2, st);
-  rc |= conv_fwd(32, 32, h->g_d2, h->conv[D2B].wb, nullptr, h->g_a4, D2, H2, W2, false, st);
-  relu_bwd(h->g_a4, h->a4, n2 * 32, st);
-  rc |= conv_wgrad(h, h->conv[D2A], h->u2, h->g_a4, D2, H2, W2, st);
-  rc |= conv_fwd(32, 96, h->g_a4, h->conv[D2A].wb, nullptr, h->g_u2, D2, H2, W2, false, st);
-  hipLaunchKernelGGL(k_upcat_bwd_coarse, dim3(grid1d(n3 * 64)), dim3(256), 0, st, h->g_u2, h->g_b3, D2, H2, W2, 64,
-                     32);
-  hipLaunchKernelGGL(k_upcat_bwd_skip, dim3(grid1d(n2 * 32)), dim3(256), 0, st, h->g_u2, h->g_s2, n2, 64, 32);
+  rc |= conv_wgrad(h->conv[D2B], h->a4, h->g_d2, D2, H2, W2, st);
+  rc |= dgrad(D2B, h->g_d2, h->a4, h->g_a4, D2, H2, W2);
+  rc |= conv_wgrad(h->conv[D2A], h->u2, h->g_a4, D2, H2, W2, st);
+  rc |= dgrad(D2A, h->g_a4, nullptr, h->g_u2, D2, H2, W2);
+  hipLaunchKernelGGL(k_upcat_bwd_coarse, dim3(grid1d(n3 * 8)), dim3(256), 0, st, h->g_u2, h->b3, h->g_b3, D2, H2, W2,
+                     64, 32);
   // bottom
-  relu_bwd(h->g_b3, h->b3, n3 * 64, st);
-  rc |= conv_wgrad(h, h->conv[B3B], h->a3, h->g_b3, D3, H3, W3, st);
-  rc |= conv_fwd(64, 64, h->g_b3, h->conv[B3B].wb, nullptr, h->g_a3, D3, H3, W3, false, st);
-  relu_bwd(h->g_a3, h->a3, n3 * 64, st);
-  rc |= conv_wgrad(h, h->conv[B3A], h->p2, h->g_a3, D3, H3, W3, st);
-  rc |= conv_fwd(64, 32, h->g_a3, h->conv[B3A].wb, nullptr, h->g_p2, D3, H3, W3, false, st);
-  hipLaunchKernelGGL(k_pool2_bwd, dim3(grid1d(n2 * 32)), dim3(256), 0, st, h->g_p2, h->g_s2, D2, H2, W2, 32, 1);
+  rc |= conv_wgrad(h->conv[B3B], h->a3, h->g_b3, D3, H3, W3, st);
+  rc |= dgrad(B3B, h->g_b3, h->a3, h->g_a3, D3, H3, W3);
+  rc |= conv_wgrad(h->conv[B3A], h->p2, h->g_a3, D3, H3, W3, st);
+  rc |= dgrad(B3A, h->g_a3, nullptr, h->g_p2, D3, H3, W3);
+  hipLaunchKernelGGL(k_skip_pool_bwd, dim3(grid1d(n2 * 4)), dim3(256), 0, st, h->g_u2, h->g_p2, h->s2, h->g_s2, D2, H2,
+                     W2, 64, 32);
   // level 2 encoder
-  relu_bwd(h->g_s2, h->s2, n2 * 32, st);
-  rc |= conv_wgrad(h, h->conv[E2B], h->a2, h->g_s2, D2, H2, W2, st);
-  rc |= conv_fwd(32, 32, h->g_s2, h->conv[E2B].wb, nullptr, h->g_a2, D2, H2, W2, false, st);
-  relu_bwd(h->g_a2, h->a2, n2 * 32, st);
-  rc |= conv_wgrad(h, h->conv[E2A], h->p1, h->g_a2, D2, H2, W2, st);
-  rc |= conv_fwd(32, 16, h->g_a2, h->conv[E2A].wb, nullptr, h->g_p1, D2, H2, W2, false, st);
-  hipLaunchKernelGGL(k_pool2_bwd, dim3(grid1d(n1 * 16)), dim3(256), 0, st, h->g_p1, h->g_s1, D, H, W, 16, 1);
+  rc |= conv_wgrad(h->conv[E2B], h->a2, h->g_s2, D2, H2, W2, st);
+  rc |= dgrad(E2B, h->g_s2, h->a2, h->g_a2, D2, H2, W2);
+  rc |= conv_wgrad(h->conv[E2A], h->p1, h->g_a2, D2, H2, W2, st);
+  rc |= dgrad(E2A, h->g_a2, nullptr, h->g_p1, D2, H2, W2);
+  hipLaunchKernelGGL(k_skip_pool_bwd, dim3(grid1d(n1 * 2)), dim3(256), 0, st, h->g_u1, h->g_p1, h->s1, h->g_s1, D, H,
+                     W, 32, 16);
   // level 1 encoder
-  relu_bwd(h->g_s1, h->s1, n1 * 16, st);
-  rc |= conv_wgrad(h, h->conv[E1B], h->a1, h->g_s1, D, H, W, st);
-  rc |= conv_fwd(16, 16, h->g_s1, h->conv[E1B].wb, nullptr, h->g_a1, D, H, W, false, st);
-  relu_bwd(h->g_a1, h->a1, n1 * 16, st);
-  rc |= conv_wgrad(h, h->conv[E1A], h->x0, h->g_a1, D, H, W, st);
+  rc |= conv_wgrad(h->conv[E1B], h->a1, h->g_s1, D, H, W, st);
+  rc |= dgrad(E1B, h->g_s1, h->a1, h->g_a1, D, H, W);
+  rc |= conv_wgrad(h->conv[E1A], h->x0, h->g_a1, D, H, W, st);
   if (rc != HFSI_OK) return rc;
+  ConvLayers tab;
+  const int blocks = conv_layers(h, tab, [](const UConv& L) { return kWgTaps * L.cout * L.cin / kGradReduceValues; });
+  hipLaunchKernelGGL(k_grad_reduce, dim3(blocks), dim3(256), 0, st, tab, h->grads);
   HFSI_LAUNCH_CHECK();
   return HFSI_OK;
 }

@@ -18,7 +18,7 @@
 // The data gradient is the same convolution of dy with the flipped, transposed
 // weights W'[ci][tap' * COUT + co] = W[co][(26 - tap') * CIN + ci]; the weight
 // gradient dW[co][tap][ci] = sum_v dy[v][co] x[v + off(tap)][ci] is an MFMA
-// GEMM with K = voxels, both operands transposed through LDS.
+// GEMM with K = voxels, both operands transposed on their way out of LDS.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -85,7 +85,17 @@ __device__ inline bool conv_brick_origin(int D, int H, int W, int& x0, int& y0, 
   return true;
 }
 
-// y[v * ycs + yoff + co] = act(bias[co] + conv(x)[v][co]); bias may be null.
+// g where y > 0, else 0: the ReLU's backward through its stored output.
+__device__ inline bf16x8 relu_gate(bf16x8 g, bf16x8 y) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    if (!((float)y[e] > 0.0f)) g[e] = (bf16)0.0f;
+  return g;
+}
+
+// y[v * ycs + yoff + co] = act(bias[co] + conv(x)[v][co]); bias may be null.  With a gate (the
+// activation that the result is the gradient of, laid out like y) the ReLU's backward is applied at
+// the store: the gradient would otherwise be read and written once more.
 //
 // The workgroup stages its tile's input with a one-voxel halo (10 x 10 x 6 voxels) in LDS,
 // CC channels at a time (conv_chunk), with 16-byte loads that follow the channels-last
@@ -103,7 +113,8 @@ __host__ __device__ constexpr int conv_chunk(int) { return 16; }
 
 template <int CIN, int COUT, bool RELU>
 __global__ void __launch_bounds__(kConvThreads) k_conv3_fwd(const bf16* __restrict__ x, const bf16* __restrict__ wt,
-                                                             const float* __restrict__ bias, bf16* __restrict__ y,
+                                                             const float* __restrict__ bias,
+                                                             const bf16* __restrict__ gate, bf16* __restrict__ y,
                                                              int ycs, int yoff, int D, int H, int W) {
   static_assert(CIN % 8 == 0 && COUT % 16 == 0, "channel counts");
   constexpr int CC = conv_chunk(CIN);
@@ -198,164 +209,226 @@ __global__ void __launch_bounds__(kConvThreads) k_conv3_fwd(const bf16* __restri
     for (int h = 0; h < 2; ++h) {
       const int q = lane;  // voxel of the wave's brick: z-slice q / 16, row q % 16 = 4 g' + i'
       const int ox = bx0 + (q & 3), oy = by0 + ((q >> 2) & 3), oz = bz0 + (q >> 4);
-      const bf16x8 v8 = *reinterpret_cast<const bf16x8*>(stage + q * 16 + 8 * h);
+      bf16x8 v8 = *reinterpret_cast<const bf16x8*>(stage + q * 16 + 8 * h);
       if (ox < W && oy < H && oz < D) {
         const long v = ((long)oz * H + oy) * W + ox;
+        if (gate) v8 = relu_gate(v8, *reinterpret_cast<const bf16x8*>(gate + v * ycs + yoff + nt * 16 + 8 * h));
         *reinterpret_cast<bf16x8*>(y + v * ycs + yoff + nt * 16 + 8 * h) = v8;
       }
     }
   }
 }
 
-// Weight gradient, per (voxel chunk, tap): partial[chunk][tap][co][ci] =
-// sum over the chunk of dy[v][co] x[v + off(tap)][ci].  Each 128-voxel step
-// stages dy and the shifted x transposed ([channel][voxel]) in LDS.
-constexpr int kWgStep = 128;
+// Weight and bias gradient: dW[co][tap][ci] = sum_v dy[v][co] x[v + off(tap)][ci] for 16 input
+// channels (blockIdx.y), with the bias as a 28th tap whose x is 1 everywhere.
+//
+// An MFMA GEMM with K = voxels.  A workgroup walks a run of 8 x 8 x 4 tiles; a tile's dy and its x
+// with a one-voxel halo are staged channels-last, as they lie in memory, and ds_read_tr16_b64 hands
+// each lane the four voxels of its channel that an operand needs (lane i of a 16-lane group gives the
+// address of voxel i / 4, channels 4 (i % 4) .. + 3 and receives channel i of the four voxels), so
+// nothing is transposed by hand and every tap of a tile is one LDS offset.  A K block is 32 voxels
+// (rows y of 8 voxels, one per lane group); a wave takes 7 of the 28 taps, its accumulators staying in
+// registers over all its tiles, and the next tile's loads are in flight while one is summed.
+// Reading x and dy once per tap from L2 and transposing them through LDS with 2-byte writes, the
+// 16 x 16 gradient took 69 us at 64^3 and the 48 x 16 one 227 us, and a bias pass 67 us more; now
+// 17.8 and 47.9 us with the bias.
+constexpr int kWgTaps = 28, kWgWaveTaps = 7;
+constexpr int kWgVox = kConvTileX * kConvTileY * kConvTileZ;  // 256
+
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+
+// Channel (lane % 16) of the 8 voxels p, p + 16, .. p + 112 bf16 (x neighbours of one row).
+__device__ inline bf16x8 read_tr8(const bf16* p) {
+  const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p);
+  const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p + 64));
+  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// Workgroups per 16 input channels: enough for one per CU over all channel blocks (two at sizes where
+// the partial sums are small beside the tiles), a multiple of HFSI_NXCD where there are that many tiles.
+__host__ __device__ inline int wgrad_parts(int tiles, int cin) {
+  const int want = (tiles >= 4096 ? 512 : 256) / (cin / 16);
+  if (tiles < HFSI_NXCD) return tiles;
+  const int n = tiles < want ? tiles : want;
+  return n / HFSI_NXCD * HFSI_NXCD;
+}
 
 template <int CIN, int COUT>
 __global__ void __launch_bounds__(kConvThreads) k_conv3_wgrad(const bf16* __restrict__ x, const bf16* __restrict__ dy,
-                                                               float* __restrict__ partial, int D, int H, int W,
-                                                               int chunk) {
+                                                               float* __restrict__ partial, int D, int H, int W) {
   static_assert(CIN % 16 == 0 && COUT % 16 == 0, "channel counts");
-  constexpr int MT = COUT / 16, NTC = CIN / 16, TILES = MT * NTC;
-  constexpr int TPW = (TILES + 3) / 4;  // tiles per wave
-  __shared__ __attribute__((aligned(16))) bf16 sdy[COUT][kWgStep];
-  __shared__ __attribute__((aligned(16))) bf16 sx[CIN][kWgStep];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const int tap = blockIdx.y;
-  int dz, dyo, dx;
-  tap_offset(tap, dz, dyo, dx);
-  const long nvox = (long)D * H * W;
-  const long vbeg = (long)blockIdx.x * chunk;
-  const long vend = vbeg + chunk < nvox ? vbeg + chunk : nvox;
-  f32x4 acc[TPW];
+  constexpr int MT = COUT / 16;
+  constexpr int XU = (kConvHaloVox * 2 + kConvThreads - 1) / kConvThreads;  // 16-byte units per thread
+  constexpr int YU = kWgVox * (COUT / 8) / kConvThreads;
+  __shared__ __attribute__((aligned(16))) bf16 sx[kConvHaloVox * 16];
+  __shared__ __attribute__((aligned(16))) bf16 sdy[MT * kWgVox * 16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, i = lane & 15;
+  const int cb = 16 * blockIdx.y, parts = gridDim.x, b = blockIdx.x;
+  const int part = parts % HFSI_NXCD == 0 ? (b % HFSI_NXCD) * (parts / HFSI_NXCD) + b / HFSI_NXCD : b;
+  const int gx = (W + kConvTileX - 1) / kConvTileX, gz = (D + kConvTileZ - 1) / kConvTileZ;
+  const long tiles = conv_tiles(D, H, W);
+  const int tbeg = (int)(tiles * part / parts), tend = (int)(tiles * (part + 1) / parts);
+  f32x4 acc[kWgWaveTaps][MT];
 #pragma unroll
-  for (int t = 0; t < TPW; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (long vs = vbeg; vs < vend; vs += kWgStep) {
-    __syncthreads();  // previous step's LDS reads are done
-    // stage dy: COUT/8 vectors per voxel
-    for (int idx = threadIdx.x; idx < kWgStep * (COUT / 8); idx += blockDim.x) {
-      const int t = idx / (COUT / 8), cv = idx % (COUT / 8);
-      const long v = vs + t;
-      bf16x8 val = bf16x8_zero();
-      if (v < vend) val = *reinterpret_cast<const bf16x8*>(dy + v * COUT + cv * 8);
+  for (int j = 0; j < kWgWaveTaps; ++j)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sdy[cv * 8 + e][t] = val[e];
+    for (int mt = 0; mt < MT; ++mt) acc[j][mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  bf16x8 rx[XU], ry[YU];
+  auto load = [&](int t) {
+    const int column = t / gz;
+    const int x0 = (column % gx) * kConvTileX, y0 = (column / gx) * kConvTileY, z0 = (t % gz) * kConvTileZ;
+#pragma unroll
+    for (int q = 0; q < XU; ++q) {
+      const int p = tid + q * kConvThreads, v = p >> 1;
+      const int xx = x0 - 1 + v % kConvHaloX, yy = y0 - 1 + (v / kConvHaloX) % kConvHaloY,
+                zz = z0 - 1 + v / (kConvHaloX * kConvHaloY);
+      rx[q] = bf16x8_zero();
+      if (v < kConvHaloVox && xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D)
+        rx[q] = *reinterpret_cast<const bf16x8*>(x + (((long)zz * H + yy) * W + xx) * CIN + cb + 8 * (p & 1));
     }
-    // stage the shifted input
-    for (int idx = threadIdx.x; idx < kWgStep * (CIN / 8); idx += blockDim.x) {
-      const int t = idx / (CIN / 8), cv = idx % (CIN / 8);
-      const long v = vs + t;
-      bf16x8 val = bf16x8_zero();
-      if (v < vend) {
-        const int xx = (int)(v % W) + dx, yy = (int)((v / W) % H) + dyo, zz = (int)(v / ((long)W * H)) + dz;
-        if (zz >= 0 && zz < D && yy >= 0 && yy < H && xx >= 0 && xx < W)
-          val = *reinterpret_cast<const bf16x8*>(x + (((long)zz * H + yy) * W + xx) * CIN + cv * 8);
-      }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sx[cv * 8 + e][t] = val[e];
+    for (int q = 0; q < YU; ++q) {
+      const int p = tid + q * kConvThreads, v = p / (COUT / 8), u = p % (COUT / 8);
+      const int xx = x0 + (v & 7), yy = y0 + ((v >> 3) & 7), zz = z0 + (v >> 6);
+      ry[q] = bf16x8_zero();
+      if (xx < W && yy < H && zz < D)
+        ry[q] = *reinterpret_cast<const bf16x8*>(dy + (((long)zz * H + yy) * W + xx) * COUT + 8 * u);
+    }
+  };
+  bf16x8 ones;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ones[e] = (bf16)1.0f;
+  if (tbeg < tend) load(tbeg);
+  for (int t = tbeg; t < tend; ++t) {
+    __syncthreads();  // the tile before is consumed
+#pragma unroll
+    for (int q = 0; q < XU; ++q) {
+      const int p = tid + q * kConvThreads;
+      if (p < 2 * kConvHaloVox) *reinterpret_cast<bf16x8*>(sx + 8 * p) = rx[q];
+    }
+#pragma unroll
+    for (int q = 0; q < YU; ++q) {
+      const int p = tid + q * kConvThreads, v = p / (COUT / 8), u = p % (COUT / 8);
+      *reinterpret_cast<bf16x8*>(sdy + ((u >> 1) * kWgVox + v) * 16 + 8 * (u & 1)) = ry[q];
     }
     __syncthreads();
+    if (t + 1 < tend) load(t + 1);
+#pragma unroll 2
+    for (int kb = 0; kb < kWgVox / 32; ++kb) {
+      const int z = kb >> 1, y = 4 * (kb & 1) + g, xv = i >> 2, c = 4 * (i & 3);
+      const bf16* a0 = sdy + ((z * kConvTileY + y) * kConvTileX + xv) * 16 + c;
+      const bf16* b0 = sx + (((z + 1) * kConvHaloY + y + 1) * kConvHaloX + xv + 1) * 16 + c;
+      bf16x8 a[MT];
 #pragma unroll
-    for (int kk = 0; kk < kWgStep; kk += 32) {
+      for (int mt = 0; mt < MT; ++mt) a[mt] = read_tr8(a0 + mt * kWgVox * 16);
 #pragma unroll
-      for (int t = 0; t < TPW; ++t) {
-        const int tile = wave + 4 * t;
-        if (tile < TILES) {
-          const int mt = tile / NTC, nt = tile % NTC;
-          const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sdy[mt * 16 + r][kk + 8 * g]);
-          const bf16x8 b = *reinterpret_cast<const bf16x8*>(&sx[nt * 16 + r][kk + 8 * g]);
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
-        }
+      for (int j = 0; j < kWgWaveTaps; ++j) {
+        const int tap = wave * kWgWaveTaps + j;
+        int dz, dyo, dx;
+        tap_offset(tap, dz, dyo, dx);
+        const bf16x8 bt = tap < 27 ? read_tr8(b0 + ((dz * kConvHaloY + dyo) * kConvHaloX + dx) * 16) : ones;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], bt, acc[j][mt], 0, 0, 0);
       }
     }
   }
-  float* out = partial + ((size_t)blockIdx.x * 27 + tap) * COUT * CIN;
+  float* out = partial + ((size_t)blockIdx.y * parts + part) * kWgTaps * COUT * 16;
 #pragma unroll
-  for (int t = 0; t < TPW; ++t) {
-    const int tile = wave + 4 * t;
-    if (tile < TILES) {
-      const int mt = tile / NTC, nt = tile % NTC;
+  for (int j = 0; j < kWgWaveTaps; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) out[(mt * 16 + 4 * g + i) * CIN + nt * 16 + r] = acc[t][i];
-    }
-  }
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        out[((wave * kWgWaveTaps + j) * COUT + mt * 16 + 4 * g + e) * 16 + i] = acc[j][mt][e];
 }
 
-// grad[co][tap * cin + ci] += sum over chunks of partial[chunk][tap][co][ci]
-__global__ void k_wgrad_reduce(const float* __restrict__ partial, int nchunks, int cin, int cout,
-                               float* __restrict__ grad) {
-  const int n = 27 * cin * cout;
-  for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += gridDim.x * blockDim.x) {
-    const int ci = idx % cin;
-    const int co = (idx / cin) % cout;
-    const int tap = idx / (cin * cout);
-    double s = 0.0;
-    for (int c = 0; c < nchunks; ++c) s += (double)partial[((size_t)c * 27 + tap) * cout * cin + co * cin + ci];
-    grad[(size_t)co * 27 * cin + tap * cin + ci] += (float)s;
-  }
+// One convolution layer of the passes over all layers (k_grad_reduce, k_conv_weights).
+struct ConvLayer {
+  int cin, cout, parts;
+  int first;              // first workgroup of the layer
+  const float* partial;   // [cin / 16][parts][28][cout][16]
+  size_t w_off, b_off;    // into the parameter vector
+  bf16 *wf, *wb;          // working weights
+};
+constexpr int kConvLayers = 10;
+struct ConvLayers {
+  ConvLayer l[kConvLayers];
+};
+
+__device__ inline int conv_layer_of(const ConvLayers& t, int block) {
+  int l = 0;
+  while (l + 1 < kConvLayers && block >= t.l[l + 1].first) ++l;
+  return l;
 }
 
-// Bias gradient partials: partial[block][co] = sum of dy[v][co] over the block's voxels.
-template <int COUT>
-__global__ void __launch_bounds__(256) k_bias_grad(const bf16* __restrict__ dy, long nvox, float* __restrict__ partial) {
-  __shared__ float red[256 / COUT][COUT];
-  const int co = threadIdx.x % COUT, lanegrp = threadIdx.x / COUT;
-  float s = 0.0f;
-  for (long v = (long)blockIdx.x * (256 / COUT) + lanegrp; v < nvox; v += (long)gridDim.x * (256 / COUT))
-    s += (float)dy[v * COUT + co];
-  red[lanegrp][co] = s;
-  __syncthreads();
-  if (threadIdx.x < COUT) {
-    float t = 0.0f;
-    for (int q = 0; q < 256 / COUT; ++q) t += red[q][threadIdx.x];
-    partial[(size_t)blockIdx.x * COUT + threadIdx.x] = t;
-  }
-}
-
-__global__ void k_bias_reduce(const float* __restrict__ partial, int nblocks, int cout, float* __restrict__ grad) {
-  const int co = threadIdx.x;
-  if (co >= cout) return;
+// grads += the partial sums of every layer, added in order in float64: 64 values per workgroup, four
+// threads each taking a quarter of the parts.
+constexpr int kGradReduceValues = 64;
+__global__ void __launch_bounds__(256) k_grad_reduce(ConvLayers tab, float* __restrict__ grads) {
+  __shared__ double part[4][kGradReduceValues];
+  const ConvLayer& L = tab.l[conv_layer_of(tab, blockIdx.x)];
+  const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int idx = (blockIdx.x - L.first) * kGradReduceValues + lane;  // a multiple of 64 values per layer
+  const int block = kWgTaps * L.cout * 16, cblk = idx / block, rem = idx % block;
+  const int tap = rem / (L.cout * 16), co = rem / 16 % L.cout, ci = rem % 16;
+  const float* src = L.partial + (size_t)cblk * L.parts * block + rem;
+  const int n0 = L.parts * q / 4, n1 = L.parts * (q + 1) / 4;
   double s = 0.0;
-  for (int b = 0; b < nblocks; ++b) s += (double)partial[(size_t)b * cout + co];
-  grad[co] += (float)s;
+#pragma unroll 8
+  for (int p = n0; p < n1; ++p) s += (double)src[(size_t)p * block];
+  part[q][lane] = s;
+  __syncthreads();
+  if (q != 0) return;
+  const float sum = (float)(((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane]);
+  if (tap < 27) grads[L.w_off + ((size_t)co * 27 + tap) * L.cin + cblk * 16 + ci] += sum;
+  else if (cblk == 0 && ci == 0) grads[L.b_off + co] += sum;
 }
 
-// dy *= (y > 0)   (ReLU backward through the stored post-activation output)
-__global__ void k_relu_bwd(bf16* __restrict__ dy, const bf16* __restrict__ y, long n) {
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    if (!((float)y[i] > 0.0f)) dy[i] = (bf16)0.0f;
-}
-
-// 2x2x2 average pooling (even fine dims): y[D/2][H/2][W/2][C]
+// 2x2x2 average pooling (even fine dims): y[D/2][H/2][W/2][C], 8 channels per thread.
 __global__ void k_pool2_fwd(const bf16* __restrict__ x, bf16* __restrict__ y, int D, int H, int W, int C) {
-  const int d = D / 2, hh = H / 2, w = W / 2;
-  const long n = (long)d * hh * w * C;
+  const int d = D / 2, hh = H / 2, w = W / 2, U = C / 8;
+  const long n = (long)d * hh * w * U;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int c = (int)(i % C);
-    const long v = i / C;
+    const int u = (int)(i % U);
+    const long v = i / U;
     const int X = (int)(v % w), Y = (int)((v / w) % hh), Z = (int)(v / ((long)w * hh));
-    float s = 0.0f;
-    for (int oz = 0; oz < 2; ++oz)
-      for (int oy = 0; oy < 2; ++oy)
-        for (int ox = 0; ox < 2; ++ox)
-          s += (float)x[((((long)(2 * Z + oz) * H) + (2 * Y + oy)) * W + (2 * X + ox)) * C + c];
-    y[i] = (bf16)(0.125f * s);
+    bf16x8 in[8];
+#pragma unroll
+    for (int o = 0; o < 8; ++o)
+      in[o] = *reinterpret_cast<const bf16x8*>(
+          x + ((((long)(2 * Z + (o >> 2)) * H) + (2 * Y + ((o >> 1) & 1))) * W + (2 * X + (o & 1))) * C + 8 * u);
+    bf16x8 out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float s = 0.0f;
+#pragma unroll
+      for (int o = 0; o < 8; ++o) s += (float)in[o][e];
+      out[e] = (bf16)(0.125f * s);
+    }
+    *reinterpret_cast<bf16x8*>(y + v * C + 8 * u) = out;
   }
 }
 
-// dx[fine] (=|+=) dy[parent] / 8
-__global__ void k_pool2_bwd(const bf16* __restrict__ dy, bf16* __restrict__ dx, int D, int H, int W, int C,
-                            int accumulate) {
-  const long n = (long)D * H * W * C;
-  const int hh = H / 2, w = W / 2;
+// Gradient of an encoder level's output y[v][0:C]: its skip part dout[v][CC + c] (dout has CC + C
+// channels) plus the pooled path dy[parent][c] / 8, through the ReLU of y.
+__global__ void k_skip_pool_bwd(const bf16* __restrict__ dout, const bf16* __restrict__ dy, const bf16* __restrict__ y,
+                                bf16* __restrict__ g, int D, int H, int W, int CC, int C) {
+  const int U = C / 8, hh = H / 2, w = W / 2;
+  const long n = (long)D * H * W * U;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int c = (int)(i % C);
-    const long v = i / C;
+    const int u = (int)(i % U);
+    const long v = i / U;
     const int X = (int)(v % W), Y = (int)((v / W) % H), Z = (int)(v / ((long)W * H));
-    const float g = 0.125f * (float)dy[((((long)(Z / 2) * hh) + Y / 2) * w + X / 2) * C + c];
-    dx[i] = (bf16)(accumulate ? (float)dx[i] + g : g);
+    const bf16x8 skip = *reinterpret_cast<const bf16x8*>(dout + v * (CC + C) + CC + 8 * u);
+    const bf16x8 up = *reinterpret_cast<const bf16x8*>(dy + ((((long)(Z / 2) * hh) + Y / 2) * w + X / 2) * C + 8 * u);
+    bf16x8 out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out[e] = (bf16)((float)skip[e] + 0.125f * (float)up[e]);
+    *reinterpret_cast<bf16x8*>(g + v * C + 8 * u) =
+        relu_gate(out, *reinterpret_cast<const bf16x8*>(y + v * C + 8 * u));
   }
 }
 
@@ -380,32 +453,31 @@ __global__ void k_upcat_fwd(const bf16* __restrict__ coarse, const bf16* __restr
   }
 }
 
-// dcoarse[p][c] = sum of the 8 children's dout[v][c] (c < CC); dskip[v][c] += dout[v][CC + c]
-__global__ void k_upcat_bwd_coarse(const bf16* __restrict__ dout, bf16* __restrict__ dcoarse, int D, int H, int W,
-                                   int CC, int CS) {
-  const int C = CC + CS;
+// dcoarse[p][c] = sum of the 8 children's dout[v][c] (c < CC) through the ReLU of the coarse output y.
+__global__ void k_upcat_bwd_coarse(const bf16* __restrict__ dout, const bf16* __restrict__ y,
+                                   bf16* __restrict__ dcoarse, int D, int H, int W, int CC, int CS) {
+  const int C = CC + CS, U = CC / 8;
   const int d = D / 2, hh = H / 2, w = W / 2;
-  const long n = (long)d * hh * w * CC;
+  const long n = (long)d * hh * w * U;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int c = (int)(i % CC);
-    const long p = i / CC;
+    const int u = (int)(i % U);
+    const long p = i / U;
     const int X = (int)(p % w), Y = (int)((p / w) % hh), Z = (int)(p / ((long)w * hh));
-    float s = 0.0f;
-    for (int oz = 0; oz < 2; ++oz)
-      for (int oy = 0; oy < 2; ++oy)
-        for (int ox = 0; ox < 2; ++ox)
-          s += (float)dout[((((long)(2 * Z + oz) * H) + (2 * Y + oy)) * W + (2 * X + ox)) * C + c];
-    dcoarse[i] = (bf16)s;
-  }
-}
-
-__global__ void k_upcat_bwd_skip(const bf16* __restrict__ dout, bf16* __restrict__ dskip, long nvox, int CC, int CS) {
-  const int C = CC + CS;
-  const long n = nvox * CS;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const long v = i / CS;
-    const int c = (int)(i % CS);
-    dskip[i] = (bf16)((float)dskip[i] + (float)dout[v * C + CC + c]);
+    bf16x8 in[8];
+#pragma unroll
+    for (int o = 0; o < 8; ++o)
+      in[o] = *reinterpret_cast<const bf16x8*>(
+          dout + ((((long)(2 * Z + (o >> 2)) * H) + (2 * Y + ((o >> 1) & 1))) * W + (2 * X + (o & 1))) * C + 8 * u);
+    bf16x8 out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float s = 0.0f;
+#pragma unroll
+      for (int o = 0; o < 8; ++o) s += (float)in[o][e];
+      out[e] = (bf16)s;
+    }
+    *reinterpret_cast<bf16x8*>(dcoarse + p * CC + 8 * u) =
+        relu_gate(out, *reinterpret_cast<const bf16x8*>(y + p * CC + 8 * u));
   }
 }
 
@@ -421,7 +493,7 @@ __global__ void k_out_fwd(const bf16* __restrict__ u, const float* __restrict__ 
   }
 }
 
-// Output layer backward: du[v][c] = dy[v] w[c]; partials of (sum_v dy u[v][c], sum_v dy).
+// Output layer backward: du[v][c] = dy[v] w[c] through the ReLU of u; partials of (sum_v dy u[v][c], sum_v dy).
 template <int CU>
 __global__ void __launch_bounds__(256) k_out_bwd(const bf16* __restrict__ u, const float* __restrict__ w,
                                                  const float* __restrict__ dyv, bf16* __restrict__ du, long nvox,
@@ -436,7 +508,7 @@ __global__ void __launch_bounds__(256) k_out_bwd(const bf16* __restrict__ u, con
     for (int c = 0; c < CU; ++c) {
       const float uc = (float)u[v * CU + c];
       acc[c] += (double)(g * uc);
-      du[v * CU + c] = (bf16)(g * w[c]);
+      du[v * CU + c] = (bf16)(uc > 0.0f ? g * w[c] : 0.0f);
     }
     acc[CU] += (double)g;
   }
@@ -480,16 +552,20 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
   }
 }
 
-// bf16 working weights of a conv layer from its float32 master [cout][27 cin]:
+// bf16 working weights of every conv layer from its float32 master [cout][27 cin]:
 // forward [cout][KP(cin)] and flipped-transposed [cin][KP(cout)], zero padded.
-__global__ void k_conv_weights(const float* __restrict__ wm, int cin, int cout, bf16* __restrict__ wf,
-                               bf16* __restrict__ wb) {
+constexpr int kWeightsPerBlock = 1024;
+__global__ void __launch_bounds__(256) k_conv_weights(ConvLayers tab, const float* __restrict__ params) {
+  const ConvLayer& L = tab.l[conv_layer_of(tab, blockIdx.x)];
+  const float* wm = params + L.w_off;
+  const int cin = L.cin, cout = L.cout;
   const int kpf = conv_kp(cin), kpb = conv_kp(cout);
-  const int nf = cout * kpf, nb = wb ? cin * kpb : 0;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nf + nb; i += gridDim.x * blockDim.x) {
+  const int nf = cout * kpf, nb = L.wb ? cin * kpb : 0;
+  const int base = (blockIdx.x - L.first) * kWeightsPerBlock;
+  for (int i = base + threadIdx.x; i < min(nf + nb, base + kWeightsPerBlock); i += blockDim.x) {
     if (i < nf) {
       const int co = i / kpf, k = i % kpf;
-      wf[i] = (bf16)(k < 27 * cin ? wm[(size_t)co * 27 * cin + k] : 0.0f);
+      L.wf[i] = (bf16)(k < 27 * cin ? wm[(size_t)co * 27 * cin + k] : 0.0f);
     } else {
       const int j = i - nf;
       const int ci = j / kpb, k = j % kpb;
@@ -498,7 +574,7 @@ __global__ void k_conv_weights(const float* __restrict__ wm, int cin, int cout, 
         const int tapb = k / cout, co = k % cout;
         val = wm[(size_t)co * 27 * cin + (26 - tapb) * cin + ci];
       }
-      wb[j] = (bf16)val;
+      L.wb[j] = (bf16)val;
     }
   }
 }

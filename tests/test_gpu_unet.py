@@ -256,3 +256,41 @@ def test_adam_first_step_closed_form_and_training_reduces_loss():
     _say(f"  loss {losses[0]:.3f} -> {losses[-1]:.3f}")
     assert losses[-1] < 0.9 * losses[0]
     L.hfsi_unet_destroy(h)
+
+
+@pytest.mark.parametrize("shape", [(4, 4, 4), (8, 20, 12), (12, 4, 40)])
+def test_gradients_at_tile_edges(shape):
+    """Weight and bias gradients where the 8 x 8 x 4 voxel tiles are cut by the grid on one, two or three
+    axes and where there are fewer tiles than XCDs, and their accumulation over two backward passes
+    (twice the single gradient, exactly: the sums are deterministic).  Tolerance as in
+    test_gradients_match_cpu_autograd."""
+    _say(f"unet gradients at {shape}")
+    _lib, L, h, params, stream = _setup(shape, 21)
+    x5 = _inputs(shape, 22)
+    rng = np.random.default_rng(23)
+    dy = rng.normal(size=shape).astype(np.float32)
+    xin, dt = torch.from_numpy(x5).cuda(), torch.from_numpy(dy).cuda()
+    y = torch.zeros(shape, dtype=torch.float32, device="cuda")
+    grads = []
+    _ok(L, L.hfsi_unet_zero_grads(h, stream))
+    _ok(L, L.hfsi_unet_forward(h, xin.data_ptr(), y.data_ptr(), stream))
+    for _ in range(2):
+        _ok(L, L.hfsi_unet_backward(h, dt.data_ptr(), stream))
+        g = np.zeros_like(params)
+        _ok(L, L.hfsi_unet_get_grads(h, g.ctypes.data, stream))
+        grads.append(g)
+    np.testing.assert_array_equal(grads[1], np.float32(2.0) * grads[0])
+    x = torch.zeros((1, 16) + shape, dtype=torch.float64)
+    x[0, :5] = _bf16(x5).permute(3, 0, 1, 2)
+    cp = _cpu_params(params, grad=True)
+    (_cpu_net(cp, x)[0] * torch.from_numpy(dy.astype(np.float64))).sum().backward()
+    gsplit = _split(grads[0].astype(np.float64))
+    for name, cin, cout in LAYERS + [("OUT", 16, 1)]:
+        for got, ref in zip(gsplit[name], cp[name]):
+            ref = ref.grad.numpy()
+            if name == "E1A" and got.ndim == 5:
+                got, ref = got[:, :5], ref[:, :5]
+            err = np.linalg.norm(got - ref) / max(np.linalg.norm(ref), 1e-30)
+            _say(f"  {name} {got.shape}: {err:.2e}")
+            assert err < 3e-2, (name, err)
+    L.hfsi_unet_destroy(h)
