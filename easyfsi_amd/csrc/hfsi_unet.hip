@@ -33,8 +33,8 @@ static_assert((int)NCONV == kConvLayers, "layer tables");
 struct UConv {
   int cin, cout, cin_true;
   size_t w_off, b_off;
-  bf16* wf = nullptr;  // forward weights [cout][KP(cin)]
-  bf16* wb = nullptr;  // data-gradient weights [cin][KP(cout)] (null for E1A)
+  bf16* wf = nullptr;  // forward weights, packed (k_conv_weights)
+  bf16* wb = nullptr;  // data-gradient weights, packed (null for E1A)
   float* partial = nullptr;  // partial weight and bias gradients of `parts` workgroups per 16 input channels
   int parts = 0;
 };
@@ -56,7 +56,7 @@ struct hfsi_unet {
   size_t w_out_off = 0, b_out_off = 0, nparams = 0;
   float *params = nullptr, *grads = nullptr, *m = nullptr, *v = nullptr;
   bf16 *x0 = nullptr, *a1 = nullptr, *s1 = nullptr, *p1 = nullptr, *a2 = nullptr, *s2 = nullptr, *p2 = nullptr,
-       *a3 = nullptr, *b3 = nullptr, *u2 = nullptr, *a4 = nullptr, *d2 = nullptr, *u1 = nullptr, *a5 = nullptr,
+       *a3 = nullptr, *b3 = nullptr, *a4 = nullptr, *d2 = nullptr, *a5 = nullptr,
        *d1 = nullptr;
   bf16 *g_a1 = nullptr, *g_s1 = nullptr, *g_p1 = nullptr, *g_a2 = nullptr, *g_s2 = nullptr, *g_p2 = nullptr,
        *g_a3 = nullptr, *g_b3 = nullptr, *g_u2 = nullptr, *g_a4 = nullptr, *g_d2 = nullptr, *g_u1 = nullptr,
@@ -84,23 +84,38 @@ static int ualloc(hfsi_unet* h, T** out, size_t count) {
 
 // ---- dispatch over the channel pairs of the topology ----------------------
 
-template <int CI, int CO>
-static void conv_fwd_t(const bf16* x, const bf16* w, const float* b, const bf16* gate, bf16* y, int D, int H, int W,
-                       bool relu, hipStream_t st) {
-  const int blocks = conv_blocks(D, H, W);
-  if (relu)
-    hipLaunchKernelGGL((k_conv3_fwd<CI, CO, true>), dim3(blocks), dim3(kConvThreads), 0, st, x, w, b, gate, y, CO, 0,
-                       D, H, W);
-  else
-    hipLaunchKernelGGL((k_conv3_fwd<CI, CO, false>), dim3(blocks), dim3(kConvThreads), 0, st, x, w, b, gate, y, CO, 0,
-                       D, H, W);
+// Workgroups per channel block: one per tile; where the weights stay in LDS, runs of tiles on at most
+// 1024 workgroups (four per CU).
+template <int CI, int CO, int NT, int ZT, bool WIDE = false>
+static void conv_launch(const ConvIn& in, const bf16* w, const float* b, const bf16* gate, bf16* y, int D, int H,
+                        int W, bool relu, hipStream_t st) {
+  int parts = conv_row_tiles(D, H, W, ZT);
+  if (conv_resident<CI, NT>() && parts > 1024) parts = 1024;
+  hipLaunchKernelGGL((k_conv3<CI, CO, NT, ZT, WIDE>), dim3(parts, CO / (16 * NT)), dim3(kConvThreads), 0, st, in, w, b, gate,
+                     y, D, H, W, relu ? 1 : 0);
 }
 
-static int conv_fwd(int ci, int co, const bf16* x, const bf16* w, const float* b, const bf16* gate, bf16* y, int D,
+// All output channels of a 16 x 4 x 4 tile per workgroup (at most 32, or 48) while that leaves a
+// workgroup for every CU.  Smaller grids are split into single rows and 16 output channels, which
+// shortens each workgroup's serial walk over the input channels (64 -> 64 at 16^3: 8.1 us with 256
+// workgroups, 40 with 16).
+template <int CI, int CO>
+static void conv_fwd_t(const ConvIn& in, const bf16* w, const float* b, const bf16* gate, bf16* y, int D, int H, int W,
+                       bool relu, hipStream_t st) {
+  constexpr int NT = CO == 16 ? 1 : CO == 48 ? 3 : 2;
+  if (conv_wide<CI>(6, H, W))
+    conv_launch<CI, CO, 1, 1, true>(in, w, b, gate, y, D, H, W, relu, st);
+  else if (conv_row_tiles(D, H, W, 4) * (CO / (16 * NT)) >= 256)
+    conv_launch<CI, CO, NT, 4>(in, w, b, gate, y, D, H, W, relu, st);
+  else
+    conv_launch<CI, CO, 1, 1>(in, w, b, gate, y, D, H, W, relu, st);
+}
+
+static int conv_fwd(int ci, int co, const ConvIn& in, const bf16* w, const float* b, const bf16* gate, bf16* y, int D,
                     int H, int W, bool relu, hipStream_t st) {
 #define HFSI_CONV_CASE(A, B)                                 \
   if (ci == A && co == B) {                                  \
-    conv_fwd_t<A, B>(x, w, b, gate, y, D, H, W, relu, st);   \
+    conv_fwd_t<A, B>(in, w, b, gate, y, D, H, W, relu, st);  \
     return HFSI_OK;                                          \
   }
   HFSI_CONV_CASE(16, 16)
@@ -125,16 +140,19 @@ static size_t wgrad_partial_size(const UConv& L, int D, int H, int W) {
 }
 
 template <int CI, int CO>
-static void conv_wgrad_t(const bf16* x, const bf16* dy, float* partial, int D, int H, int W, hipStream_t st) {
-  hipLaunchKernelGGL((k_conv3_wgrad<CI, CO>), dim3(wgrad_parts(conv_tiles(D, H, W), CI), CI / 16), dim3(kConvThreads),
-                     0, st, x, dy, partial, D, H, W);
+static void conv_wgrad_t(const ConvIn& in, const bf16* dy, float* partial, int D, int H, int W, hipStream_t st) {
+  const dim3 grid(wgrad_parts(conv_tiles(D, H, W), CI), CI / 16);
+  if (conv_wide<CI>(kConvHaloZ, H, W) || conv_wide<CO>(kConvTileZ, H, W))
+    hipLaunchKernelGGL((k_conv3_wgrad<CI, CO, true>), grid, dim3(kConvThreads), 0, st, in, dy, partial, D, H, W);
+  else
+    hipLaunchKernelGGL((k_conv3_wgrad<CI, CO, false>), grid, dim3(kConvThreads), 0, st, in, dy, partial, D, H, W);
 }
 
 // The layer's partial weight and bias gradients (summed for all layers by k_grad_reduce).
-static int conv_wgrad(const UConv& L, const bf16* x, const bf16* dy, int D, int H, int W, hipStream_t st) {
+static int conv_wgrad(const UConv& L, const ConvIn& in, const bf16* dy, int D, int H, int W, hipStream_t st) {
 #define HFSI_WGRAD_CASE(A, B)                              \
   if (L.cin == A && L.cout == B) {                         \
-    conv_wgrad_t<A, B>(x, dy, L.partial, D, H, W, st);     \
+    conv_wgrad_t<A, B>(in, dy, L.partial, D, H, W, st);    \
     return HFSI_OK;                                        \
   }
   HFSI_WGRAD_CASE(16, 16)
@@ -175,10 +193,28 @@ struct FinLoss {
   __device__ void operator()(const double*) const {}
 };
 
+// He-normal convolution weights over the true fan-in, zero biases; the padded input channels of E1A
+// start (and stay near) zero.  A function of its own: inlined into hfsi_unet_create its loop compiles
+// to calls per value (15 -> 26 ms per network).
+__attribute__((noinline)) static std::vector<float> initial_params(const hfsi_unet* h, uint64_t seed) {
+  std::vector<float> p(h->nparams, 0.0f);
+  std::mt19937_64 gen(seed);
+  for (int l = 0; l < NCONV; ++l) {
+    const UConv& L = h->conv[l];
+    std::normal_distribution<float> nd(0.0f, std::sqrt(2.0f / (27.0f * L.cin_true)));
+    float* w = p.data() + L.w_off;
+    for (int row = 0; row < L.cout * 27; ++row)
+      for (int ci = 0; ci < L.cin_true; ++ci) w[row * L.cin + ci] = nd(gen);
+  }
+  std::normal_distribution<float> no(0.0f, 0.25f);
+  for (int c = 0; c < 16; ++c) p[h->w_out_off + c] = no(gen);
+  return p;
+}
+
 static int refresh_weights(hfsi_unet* h, hipStream_t st) {
   ConvLayers tab;
   const int blocks = conv_layers(h, tab, [](const UConv& L) {
-    const int n = L.cout * conv_kp(L.cin) + (L.wb ? L.cin * conv_kp(L.cout) : 0);
+    const int n = conv_packed(L.cin, L.cout) + (L.wb ? conv_packed(L.cout, L.cin) : 0);
     return (n + kWeightsPerBlock - 1) / kWeightsPerBlock;
   });
   hipLaunchKernelGGL(k_conv_weights, dim3(blocks), dim3(256), 0, st, tab, (const float*)h->params);
@@ -237,8 +273,8 @@ int hfsi_unet_create(hfsi_unet** out, int32_t nx, int32_t ny, int32_t nz, int32_
   rc |= ualloc(h, &h->v, off);
   for (int l = 0; l < NCONV && rc == HFSI_OK; ++l) {
     UConv& L = h->conv[l];
-    rc |= ualloc(h, &L.wf, (size_t)L.cout * conv_kp(L.cin));
-    if (l != E1A) rc |= ualloc(h, &L.wb, (size_t)L.cin * conv_kp(L.cout));
+    rc |= ualloc(h, &L.wf, (size_t)conv_packed(L.cin, L.cout));
+    if (l != E1A) rc |= ualloc(h, &L.wb, (size_t)conv_packed(L.cout, L.cin));
   }
   const long n1 = h->n1, n2 = h->n2, n3 = h->n3;
   if (rc == HFSI_OK) {
@@ -251,10 +287,8 @@ int hfsi_unet_create(hfsi_unet** out, int32_t nx, int32_t ny, int32_t nz, int32_
     rc |= ualloc(h, &h->p2, n3 * 32);
     rc |= ualloc(h, &h->a3, n3 * 64);
     rc |= ualloc(h, &h->b3, n3 * 64);
-    rc |= ualloc(h, &h->u2, n2 * 96);
     rc |= ualloc(h, &h->a4, n2 * 32);
     rc |= ualloc(h, &h->d2, n2 * 32);
-    rc |= ualloc(h, &h->u1, n1 * 48);
     rc |= ualloc(h, &h->a5, n1 * 16);
     rc |= ualloc(h, &h->d1, n1 * 16);
     rc |= ualloc(h, &h->partials, 8192 * 32);
@@ -287,20 +321,7 @@ int hfsi_unet_create(hfsi_unet** out, int32_t nx, int32_t ny, int32_t nz, int32_
     rc = HFSI_ERR_HIP;
   }
   if (rc == HFSI_OK) {
-    // He-normal convolution weights over the true fan-in, zero biases; the
-    // padded input channels of E1A start (and stay near) zero.
-    std::vector<float> p(off, 0.0f);
-    std::mt19937_64 gen(seed);
-    for (int l = 0; l < NCONV; ++l) {
-      const UConv& L = h->conv[l];
-      std::normal_distribution<float> nd(0.0f, std::sqrt(2.0f / (27.0f * L.cin_true)));
-      for (int co = 0; co < L.cout; ++co)
-        for (int tap = 0; tap < 27; ++tap)
-          for (int ci = 0; ci < L.cin; ++ci)
-            p[L.w_off + ((size_t)co * 27 + tap) * L.cin + ci] = ci < L.cin_true ? nd(gen) : 0.0f;
-    }
-    std::normal_distribution<float> no(0.0f, 0.25f);
-    for (int c = 0; c < 16; ++c) p[h->w_out_off + c] = no(gen);
+    const std::vector<float> p = initial_params(h, seed);
     if (hipMemcpy(h->params, p.data(), off * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(h->grads, 0, off * sizeof(float)) != hipSuccess ||
         hipMemset(h->m, 0, off * sizeof(float)) != hipSuccess ||
@@ -388,20 +409,18 @@ int hfsi_unet_forward(hfsi_unet* h, const float* in5, float* out, void* stream) 
   auto b = [&](int l) { return P + h->conv[l].b_off; };
   hipLaunchKernelGGL(k_unet_input, dim3(grid1d(h->n1)), dim3(256), 0, st, in5, h->x0, h->n1);
   int rc = HFSI_OK;
-  rc |= conv_fwd(16, 16, h->x0, h->conv[E1A].wf, b(E1A), nullptr, h->a1, D, H, W, true, st);
-  rc |= conv_fwd(16, 16, h->a1, h->conv[E1B].wf, b(E1B), nullptr, h->s1, D, H, W, true, st);
+  rc |= conv_fwd(16, 16, ConvIn{h->x0, nullptr}, h->conv[E1A].wf, b(E1A), nullptr, h->a1, D, H, W, true, st);
+  rc |= conv_fwd(16, 16, ConvIn{h->a1, nullptr}, h->conv[E1B].wf, b(E1B), nullptr, h->s1, D, H, W, true, st);
   hipLaunchKernelGGL(k_pool2_fwd, dim3(grid1d(h->n2 * 2)), dim3(256), 0, st, h->s1, h->p1, D, H, W, 16);
-  rc |= conv_fwd(16, 32, h->p1, h->conv[E2A].wf, b(E2A), nullptr, h->a2, D2, H2, W2, true, st);
-  rc |= conv_fwd(32, 32, h->a2, h->conv[E2B].wf, b(E2B), nullptr, h->s2, D2, H2, W2, true, st);
+  rc |= conv_fwd(16, 32, ConvIn{h->p1, nullptr}, h->conv[E2A].wf, b(E2A), nullptr, h->a2, D2, H2, W2, true, st);
+  rc |= conv_fwd(32, 32, ConvIn{h->a2, nullptr}, h->conv[E2B].wf, b(E2B), nullptr, h->s2, D2, H2, W2, true, st);
   hipLaunchKernelGGL(k_pool2_fwd, dim3(grid1d(h->n3 * 4)), dim3(256), 0, st, h->s2, h->p2, D2, H2, W2, 32);
-  rc |= conv_fwd(32, 64, h->p2, h->conv[B3A].wf, b(B3A), nullptr, h->a3, D3, H3, W3, true, st);
-  rc |= conv_fwd(64, 64, h->a3, h->conv[B3B].wf, b(B3B), nullptr, h->b3, D3, H3, W3, true, st);
-  hipLaunchKernelGGL(k_upcat_fwd, dim3(grid1d(h->n2 * 12)), dim3(256), 0, st, h->b3, h->s2, h->u2, D2, H2, W2, 64, 32);
-  rc |= conv_fwd(96, 32, h->u2, h->conv[D2A].wf, b(D2A), nullptr, h->a4, D2, H2, W2, true, st);
-  rc |= conv_fwd(32, 32, h->a4, h->conv[D2B].wf, b(D2B), nullptr, h->d2, D2, H2, W2, true, st);
-  hipLaunchKernelGGL(k_upcat_fwd, dim3(grid1d(h->n1 * 6)), dim3(256), 0, st, h->d2, h->s1, h->u1, D, H, W, 32, 16);
-  rc |= conv_fwd(48, 16, h->u1, h->conv[D1A].wf, b(D1A), nullptr, h->a5, D, H, W, true, st);
-  rc |= conv_fwd(16, 16, h->a5, h->conv[D1B].wf, b(D1B), nullptr, h->d1, D, H, W, true, st);
+  rc |= conv_fwd(32, 64, ConvIn{h->p2, nullptr}, h->conv[B3A].wf, b(B3A), nullptr, h->a3, D3, H3, W3, true, st);
+  rc |= conv_fwd(64, 64, ConvIn{h->a3, nullptr}, h->conv[B3B].wf, b(B3B), nullptr, h->b3, D3, H3, W3, true, st);
+  rc |= conv_fwd(96, 32, ConvIn{h->b3, h->s2}, h->conv[D2A].wf, b(D2A), nullptr, h->a4, D2, H2, W2, true, st);
+  rc |= conv_fwd(32, 32, ConvIn{h->a4, nullptr}, h->conv[D2B].wf, b(D2B), nullptr, h->d2, D2, H2, W2, true, st);
+  rc |= conv_fwd(48, 16, ConvIn{h->d2, h->s1}, h->conv[D1A].wf, b(D1A), nullptr, h->a5, D, H, W, true, st);
+  rc |= conv_fwd(16, 16, ConvIn{h->a5, nullptr}, h->conv[D1B].wf, b(D1B), nullptr, h->d1, D, H, W, true, st);
   hipLaunchKernelGGL((k_out_fwd<16>), dim3(grid1d(h->n1)), dim3(256), 0, st, h->d1, P + h->w_out_off,
                      P + h->b_out_off, out, h->n1);
   if (rc != HFSI_OK) return rc;
@@ -431,40 +450,40 @@ int hfsi_unet_backward(hfsi_unet* h, const float* dout, void* stream) {
   // Every gradient that is written here has its ReLU applied where it is produced (gates), but those of
   // the concatenations and pooled tensors, which have none.
   auto dgrad = [&](int l, const bf16* dy, const bf16* gate, bf16* dx, int d, int hh, int w) {
-    return conv_fwd(h->conv[l].cout, h->conv[l].cin, dy, h->conv[l].wb, nullptr, gate, dx, d, hh, w, false, st);
+    return conv_fwd(h->conv[l].cout, h->conv[l].cin, ConvIn{dy, nullptr}, h->conv[l].wb, nullptr, gate, dx, d, hh, w, false, st);
   };
   // level 1 decoder
-  rc |= conv_wgrad(h->conv[D1B], h->a5, h->g_d1, D, H, W, st);
+  rc |= conv_wgrad(h->conv[D1B], ConvIn{h->a5, nullptr}, h->g_d1, D, H, W, st);
   rc |= dgrad(D1B, h->g_d1, h->a5, h->g_a5, D, H, W);
-  rc |= conv_wgrad(h->conv[D1A], h->u1, h->g_a5, D, H, W, st);
+  rc |= conv_wgrad(h->conv[D1A], ConvIn{h->d2, h->s1}, h->g_a5, D, H, W, st);
   rc |= dgrad(D1A, h->g_a5, nullptr, h->g_u1, D, H, W);
   hipLaunchKernelGGL(k_upcat_bwd_coarse, dim3(grid1d(n2 * 4)), dim3(256), 0, st, h->g_u1, h->d2, h->g_d2, D, H, W, 32,
                      16);
   // level 2 decoder
-  rc |= conv_wgrad(h->conv[D2B], h->a4, h->g_d2, D2, H2, W2, st);
+  rc |= conv_wgrad(h->conv[D2B], ConvIn{h->a4, nullptr}, h->g_d2, D2, H2, W2, st);
   rc |= dgrad(D2B, h->g_d2, h->a4, h->g_a4, D2, H2, W2);
-  rc |= conv_wgrad(h->conv[D2A], h->u2, h->g_a4, D2, H2, W2, st);
+  rc |= conv_wgrad(h->conv[D2A], ConvIn{h->b3, h->s2}, h->g_a4, D2, H2, W2, st);
   rc |= dgrad(D2A, h->g_a4, nullptr, h->g_u2, D2, H2, W2);
   hipLaunchKernelGGL(k_upcat_bwd_coarse, dim3(grid1d(n3 * 8)), dim3(256), 0, st, h->g_u2, h->b3, h->g_b3, D2, H2, W2,
                      64, 32);
   // bottom
-  rc |= conv_wgrad(h->conv[B3B], h->a3, h->g_b3, D3, H3, W3, st);
+  rc |= conv_wgrad(h->conv[B3B], ConvIn{h->a3, nullptr}, h->g_b3, D3, H3, W3, st);
   rc |= dgrad(B3B, h->g_b3, h->a3, h->g_a3, D3, H3, W3);
-  rc |= conv_wgrad(h->conv[B3A], h->p2, h->g_a3, D3, H3, W3, st);
+  rc |= conv_wgrad(h->conv[B3A], ConvIn{h->p2, nullptr}, h->g_a3, D3, H3, W3, st);
   rc |= dgrad(B3A, h->g_a3, nullptr, h->g_p2, D3, H3, W3);
   hipLaunchKernelGGL(k_skip_pool_bwd, dim3(grid1d(n2 * 4)), dim3(256), 0, st, h->g_u2, h->g_p2, h->s2, h->g_s2, D2, H2,
                      W2, 64, 32);
   // level 2 encoder
-  rc |= conv_wgrad(h->conv[E2B], h->a2, h->g_s2, D2, H2, W2, st);
+  rc |= conv_wgrad(h->conv[E2B], ConvIn{h->a2, nullptr}, h->g_s2, D2, H2, W2, st);
   rc |= dgrad(E2B, h->g_s2, h->a2, h->g_a2, D2, H2, W2);
-  rc |= conv_wgrad(h->conv[E2A], h->p1, h->g_a2, D2, H2, W2, st);
+  rc |= conv_wgrad(h->conv[E2A], ConvIn{h->p1, nullptr}, h->g_a2, D2, H2, W2, st);
   rc |= dgrad(E2A, h->g_a2, nullptr, h->g_p1, D2, H2, W2);
   hipLaunchKernelGGL(k_skip_pool_bwd, dim3(grid1d(n1 * 2)), dim3(256), 0, st, h->g_u1, h->g_p1, h->s1, h->g_s1, D, H,
                      W, 32, 16);
   // level 1 encoder
-  rc |= conv_wgrad(h->conv[E1B], h->a1, h->g_s1, D, H, W, st);
+  rc |= conv_wgrad(h->conv[E1B], ConvIn{h->a1, nullptr}, h->g_s1, D, H, W, st);
   rc |= dgrad(E1B, h->g_s1, h->a1, h->g_a1, D, H, W);
-  rc |= conv_wgrad(h->conv[E1A], h->x0, h->g_a1, D, H, W, st);
+  rc |= conv_wgrad(h->conv[E1A], ConvIn{h->x0, nullptr}, h->g_a1, D, H, W, st);
   if (rc != HFSI_OK) return rc;
   ConvLayers tab;
   const int blocks = conv_layers(h, tab, [](const UConv& L) { return kWgTaps * L.cout * L.cin / kGradReduceValues; });

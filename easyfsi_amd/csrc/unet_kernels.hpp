@@ -12,7 +12,7 @@
 // 3x3x3 convolution, zero padding, as an implicit GEMM
 //   y[v][co] = bias[co] + sum_{tap, ci} W[co][tap * CIN + ci] * x[v + off(tap)][ci]
 // with tap = (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1):
-//   M = voxels (16 per MFMA row block), N = output channels, K = 27 * CIN,
+//   M = output channels, N = voxels, K = 27 * CIN,
 //   v_mfma_f32_16x16x32_bf16: lane l holds A[l % 16][8 (l / 16) .. + 7],
 //   B[8 (l / 16) .. + 7][l % 16] and D[4 (l / 16) + i][l % 16], i < 4.
 // The data gradient is the same convolution of dy with the flipped, transposed
@@ -29,12 +29,11 @@ namespace hfsi {
 
 typedef __bf16 bf16;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef __attribute__((__vector_size__(4 * sizeof(float)), aligned(4))) float f32x4_u;
 
 constexpr int kConvThreads = 256;  // 4 waves
-constexpr int kConvVoxWave = 64;   // voxels per wave (4 MFMA row blocks)
-
-__host__ __device__ constexpr int conv_kp(int cin) { return (27 * cin + 31) / 32 * 32; }
 
 __device__ inline bf16x8 bf16x8_zero() {
   bf16x8 z;
@@ -49,40 +48,114 @@ __device__ inline void tap_offset(int tap, int& dz, int& dy, int& dx) {
   dx = tap % 3 - 1;
 }
 
-// Voxels of a convolution launch: a workgroup owns an 8 x 8 x 4 (x, y, z) tile, its wave w the
-// 4 x 4 x 4 brick at (4 (w & 1), 4 (w >> 1), 0) of it; MFMA row block mt of a wave is the brick's
-// z-slice mt and row r within it the voxel (r % 4, r / 4).  A wave's 27-tap input footprint is
-// 6 x 6 x 6 voxels.  Tiles are ordered z fastest along (x, y) columns, and workgroup b (which
-// runs on XCD b % 8) takes tile (b % 8) * (G / 8) + b / 8: each XCD walks a contiguous run of
-// columns, so the tiles in flight on one XCD are z-neighbours in adjacent columns and their taps
-// re-read inputs from that XCD's L2 instead of HBM (the 48-channel decoder input is 201 MB at
-// 128^3, read by 27 taps).  A voxel's K blocks run in the same order under any mapping; the
-// hardware's summation inside one MFMA may depend on the row, so results can differ from another
-// mapping in the last float32 bits.
-constexpr int kConvTileX = 8, kConvTileY = 8, kConvTileZ = 4;
+// Input of a convolution: CIN channels of x, or, for the two decoder convolutions that follow an
+// upsampling and concatenation (conv_cat(CIN) > 0), that many channels of the coarse tensor x at the
+// parent voxel and the rest of `skip`: the concatenation (201 MB at 128^3) is never written.
+struct ConvIn {
+  const bf16* x;
+  const bf16* skip;
+};
+__host__ __device__ constexpr int conv_cat(int cin) { return cin == 48 ? 32 : cin == 96 ? 64 : 0; }
 
-__host__ __device__ inline int conv_tiles(int D, int H, int W) {
-  return ((W + kConvTileX - 1) / kConvTileX) * ((H + kConvTileY - 1) / kConvTileY) *
-         ((D + kConvTileZ - 1) / kConvTileZ);
+// 8 channels (channel block cb of 16, half `cu`) of voxel (zz, yy, xx); zero outside the grid.
+template <int CIN>
+__device__ inline bf16x8 conv_input(const ConvIn& in, int cb, int cu, int zz, int yy, int xx, int D, int H, int W) {
+  constexpr int CC = conv_cat(CIN);
+  if (!(xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D)) return bf16x8_zero();
+  const bf16* p;
+  if (CC == 0) p = in.x + (((long)zz * H + yy) * W + xx) * CIN + cb;
+  else if (cb < CC) p = in.x + (((long)(zz >> 1) * (H >> 1) + (yy >> 1)) * (W >> 1) + (xx >> 1)) * CC + cb;
+  else p = in.skip + (((long)zz * H + yy) * W + xx) * (CIN - CC) + (cb - CC);
+  return *reinterpret_cast<const bf16x8*>(p + 8 * cu);
 }
 
-// Workgroups of a launch: the tile count rounded up to a multiple of HFSI_NXCD.
-__host__ __device__ inline int conv_blocks(int D, int H, int W) {
-  return (conv_tiles(D, H, W) + HFSI_NXCD - 1) / HFSI_NXCD * HFSI_NXCD;
+// Bytes that a tile's halo may span for its loads to use 32-bit offsets.
+constexpr long kConvSpan = 0xfffff000L;
+template <int CIN>
+__host__ __device__ inline bool conv_wide(int halo_z, int H, int W) {
+  return (long)halo_z * H * W * CIN * 2 >= kConvSpan;
 }
 
-// Origin of this wave's brick (it may lie past the grid's edge); false for the padding
-// workgroups past the last tile, for the whole workgroup alike.
-__device__ inline bool conv_brick_origin(int D, int H, int W, int& x0, int& y0, int& z0) {
-  const int gx = (W + kConvTileX - 1) / kConvTileX, gz = (D + kConvTileZ - 1) / kConvTileZ;
-  const int G = (int)gridDim.x, b = blockIdx.x, wave = threadIdx.x >> 6;
-  const int t = (b % HFSI_NXCD) * (G / HFSI_NXCD) + b / HFSI_NXCD;
-  if (t >= conv_tiles(D, H, W)) return false;
-  const int column = t / gz;
-  x0 = (column % gx) * kConvTileX + 4 * (wave & 1);
-  y0 = (column / gx) * kConvTileY + 4 * (wave >> 1);
-  z0 = (t % gz) * kConvTileZ;
-  return true;
+// A tile's input with a one-voxel halo (HX x HY x HZ voxels from (x0 - 1, y0 - 1, z0 - 1)), 16 channels
+// at a time: 16-byte unit p = voxel p / 2, half p % 2; thread t holds units t, t + 256, ...
+// Address arithmetic per load (70 instructions, a branch per boundary, 4 cycles each: 89 against 61 us
+// for 16 -> 16 at 128^3) bounds the convolutions, so each thread's offsets from the tile's corner are
+// computed once per kernel, the corner is a scalar, and buffer loads return zero for the
+// voxels outside the grid (offset ~0), which only tiles at the boundary have to look for.
+// WIDE: grids whose halos span more than 32-bit offsets reach, addressed voxel by voxel.
+template <int CIN, int HX, int HY, int HZ, bool WIDE>
+struct HaloLoader {
+  static constexpr int CC = conv_cat(CIN), CS = CIN - CC;
+  static constexpr int kUnits = 2 * HX * HY * HZ, XU = (kUnits + kConvThreads - 1) / kConvThreads;
+  uint32_t off[XU], coarse[CC > 0 ? XU : 1], at[XU];
+
+  __device__ inline void init(int H, int W) {
+#pragma unroll
+    for (int q = 0; q < XU; ++q) {
+      const int p = threadIdx.x + q * kConvThreads, v = p >> 1;
+      const uint32_t hx = v % HX, hy = v / HX % HY, hz = v / (HX * HY);
+      const uint32_t half = 16 * (p & 1);
+      at[q] = hx | hy << 8 | hz << 16;
+      off[q] = p < kUnits ? ((hz * H + hy) * W + hx) * (CS * 2) + half : ~0u;
+      // x0 and y0 are even: the parent of corner + h is the corner's parent + (h + 1) / 2; z: see load
+      if (CC > 0) coarse[q] = (((hy + 1) >> 1) * (W >> 1) + ((hx + 1) >> 1)) * (CC * 2) + half;
+    }
+  }
+
+  // channels cb .. cb + 15 into r
+  __device__ inline void load(const ConvIn& in, int cb, int x0, int y0, int z0, int D, int H, int W,
+                              bf16x8 (&r)[XU]) const {
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int q = 0; q < XU; ++q) {
+        r[q] = bf16x8_zero();
+        if (off[q] != ~0u)
+          r[q] = conv_input<CIN>(in, cb, threadIdx.x & 1, z0 - 1 + (int)(at[q] >> 16), y0 - 1 + (int)(at[q] >> 8 & 255),
+                                 x0 - 1 + (int)(at[q] & 255), D, H, W);
+      }
+    } else {
+      const bool up = CC > 0 && cb < CC;
+      const bf16* corner =
+          up ? in.x + ((((long)(z0 >> 1) - 1) * (H >> 1) + (y0 >> 1) - 1) * (W >> 1) + (x0 >> 1) - 1) * CC + cb
+             : (CC > 0 ? in.skip : in.x) + ((((long)z0 - 1) * H + y0 - 1) * W + x0 - 1) * CS + (cb - CC);
+      const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(corner), 0, (int)(uint32_t)kConvSpan, 0x00027000);
+      const bool inner = x0 > 0 && y0 > 0 && z0 > 0 && x0 + HX - 2 < W && y0 + HY - 2 < H && z0 + HZ - 2 < D;
+      uint32_t o[XU];
+#pragma unroll
+      for (int q = 0; q < XU; ++q) {
+        o[q] = off[q];
+        if (up) {
+          const uint32_t dz = ((at[q] >> 16) + 1 + (z0 & 1)) >> 1;  // z0 may be odd where tiles are one slice
+          const uint32_t parent = coarse[CC > 0 ? q : 0] + dz * ((uint32_t)(H >> 1) * (W >> 1) * (CC * 2));
+          o[q] = off[q] == ~0u ? ~0u : parent;
+        }
+      }
+      if (!inner) {
+#pragma unroll
+        for (int q = 0; q < XU; ++q) {
+          const uint32_t xx = x0 - 1 + (at[q] & 255), yy = y0 - 1 + (at[q] >> 8 & 255), zz = z0 - 1 + (at[q] >> 16);
+          o[q] = (xx < (uint32_t)W) & (yy < (uint32_t)H) & (zz < (uint32_t)D) ? o[q] : ~0u;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < XU; ++q)
+        r[q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)o[q], 0, 0));
+    }
+  }
+};
+
+// The next tile along z, then the next column (tiles of TX x TY x TZ voxels).
+template <int TX, int TY, int TZ>
+__device__ inline void next_tile(int& x0, int& y0, int& z0, int D, int W) {
+  z0 += TZ;
+  if (z0 >= D) {
+    z0 = 0;
+    x0 += TX;
+    if (x0 >= W) {
+      x0 = 0;
+      y0 += TY;
+    }
+  }
 }
 
 // g where y > 0, else 0: the ReLU's backward through its stored output.
@@ -93,129 +166,192 @@ __device__ inline bf16x8 relu_gate(bf16x8 g, bf16x8 y) {
   return g;
 }
 
-// y[v * ycs + yoff + co] = act(bias[co] + conv(x)[v][co]); bias may be null.  With a gate (the
-// activation that the result is the gradient of, laid out like y) the ReLU's backward is applied at
-// the store: the gradient would otherwise be read and written once more.
+// y[v][co] = act(bias[co] + conv(x)[v][co]); bias may be null.  With a gate (the activation that the
+// result is the gradient of, laid out like y) the ReLU's backward is applied at the store: the
+// gradient would otherwise be read and written once more.
 //
-// The workgroup stages its tile's input with a one-voxel halo (10 x 10 x 6 voxels) in LDS,
-// CC channels at a time (conv_chunk), with 16-byte loads that follow the channels-last
-// layout (zero outside the grid: the convolution's padding).  The K dimension is then walked as
-// units of 8 channels of one tap, tap-major (unit u = tap * CC / 8 + channel group); a 32-wide
-// MFMA K block takes 4 consecutive units, which may straddle two taps, its A operand read from
-// LDS and its B operand (the weight row at tap * CIN + channel) from global memory, where the
-// weights stay cached.  Every input voxel is read from HBM / L2 about 600 / 256 times per launch
-// instead of 27 times.
-constexpr int kConvHaloX = kConvTileX + 2, kConvHaloY = kConvTileY + 2, kConvHaloZ = kConvTileZ + 2;
-constexpr int kConvHaloVox = kConvHaloX * kConvHaloY * kConvHaloZ;  // 600
+// A workgroup (4 waves) owns tiles of 16 x 4 x ZT voxels (x, y, z) and NT blocks of 16 output
+// channels; a wave ZT of the tile's 4 ZT rows of 16 voxels.  The tile's input with a one-voxel halo is
+// staged 16 channels at a time as two planes of 8 channels (16 bytes per voxel), so that an operand
+// read is 256 consecutive bytes per lane group: 8 x 8 x 4 tiles of 32-byte voxels spent 45 % of the LDS
+// cycles in bank conflicts.  A = weights (16 channels x 32), B = voxels (32 x 16): lane l ends with 4
+// consecutive channels of voxel l % 16, an 8-byte store without staging.  K: 27 taps x 2 planes = 54
+// units of 8 channels, tap-major, 4 per MFMA, padded to 56 with zeros; one accumulation chain per
+// output in that order for every tile shape (another order, as sharing an operand between the three
+// taps along x, changes which sums round to the next bf16, and through the layers and Adam's
+// normalised steps a training gradient by up to 3 %).
+// The weights come packed in operand order (k_conv_weights) and lie in LDS: all of them, loaded once,
+// where they fit (RES), else those of the current 16 channels.  The next input (of the same tile or
+// the next) is loaded while one is multiplied.  16 -> 16 at 128^3 80 -> 52 us, 48 -> 16 193 -> 142 us
+// without the 2 x 37 us of writing the concatenations, 96 -> 32 at 64^3 90 -> 56 us: the network
+// 764 -> 460 us, bit for bit the same.
+// Tiles are ordered z fastest along (x, y) columns; a workgroup takes a run of them, the runs of one
+// XCD adjacent, so that halos are re-read from that XCD's L2.
+constexpr int kConvX = 16, kConvY = 4, kConvUnits = 54, kConvIters = (kConvUnits + 3) / 4;
 
-// Channels staged per LDS chunk: 16 (a 19.2 KB tile: up to eight workgroups per CU by LDS).
-__host__ __device__ constexpr int conv_chunk(int) { return 16; }
+__host__ __device__ inline int conv_row_tiles(int D, int H, int W, int zt) {
+  return ((W + kConvX - 1) / kConvX) * ((H + kConvY - 1) / kConvY) * ((D + zt - 1) / zt);
+}
 
-template <int CIN, int COUT, bool RELU>
-__global__ void __launch_bounds__(kConvThreads) k_conv3_fwd(const bf16* __restrict__ x, const bf16* __restrict__ wt,
-                                                             const float* __restrict__ bias,
-                                                             const bf16* __restrict__ gate, bf16* __restrict__ y,
-                                                             int ycs, int yoff, int D, int H, int W) {
-  static_assert(CIN % 8 == 0 && COUT % 16 == 0, "channel counts");
-  constexpr int CC = conv_chunk(CIN);
-  static_assert(CIN % CC == 0, "channel chunks");
-  constexpr int VS = CC;           // LDS voxel stride in bf16 (unpadded: a smaller tile, more workgroups per CU)
-  constexpr int UNITS = CC / 8;    // 8-channel units per tap and chunk
-  constexpr int KU = 27 * UNITS;   // units per chunk
-  constexpr int KP = conv_kp(CIN);
-  constexpr int NT = COUT / 16;
-  constexpr int MT = kConvVoxWave / 16;  // z-slices of the brick
-  constexpr int NIT = (KU + 3) / 4;      // 32-wide K blocks per chunk
-  constexpr int PD = NT <= 2 ? 3 : 0;    // weight prefetch distance in K blocks (wide outputs: none)
-  __shared__ __attribute__((aligned(16))) bf16 tile[kConvHaloVox * VS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int bx0 = 0, by0 = 0, bz0 = 0;
-  if (!conv_brick_origin(D, H, W, bx0, by0, bz0)) return;  // whole workgroup: before any barrier
-  const int tx0 = bx0 - 4 * (wave & 1) - 1, ty0 = by0 - 4 * (wave >> 1) - 1, tz0 = bz0 - 1;  // halo origin
-  const int r = lane & 15, g = lane >> 4;
-  // this lane's A voxel in the halo tile, z-slice 0, tap (0, 0, 0) offset (1, 1, 1)
-  const int lx = 1 + 4 * (wave & 1) + (r & 3), ly = 1 + 4 * (wave >> 1) + (r >> 2);
-  f32x4 acc[MT][NT];
+// Packed weights: [cin / 16][14 MFMAs][cout / 16][64 lanes][8], element e of lane l = output channel
+// 16 nt + l % 16 of unit u = 4 it + l / 16: tap u / 2, input channel 16 c + 8 (u % 2) + e.
+__host__ __device__ constexpr int conv_packed(int cin, int cout) { return cin / 16 * kConvIters * (cout / 16) * 512; }
+
+// All weights in LDS where they leave room for three workgroups per CU (or two with one channel block:
+// 48 -> 16 at 128^3 142 against 157 us); reloading them per 16 channels with more workgroups is the
+// better one above (32 -> 32 at 64^3 26.0 against 31.7 us, 64 -> 64 at 16^3 8.1 against 11.3).
+template <int CIN, int NT>
+__host__ __device__ constexpr bool conv_resident() {
+  constexpr int kb = CIN / 16 * kConvIters * NT;
+  return CIN == 16 || kb <= 28 || (NT == 1 && kb <= 42);
+}
+
+template <int CIN, int COUT, int NT, int ZT, bool WIDE>
+__global__ void __launch_bounds__(kConvThreads) k_conv3(ConvIn in, const bf16* __restrict__ wt,
+                                                         const float* __restrict__ bias, const bf16* __restrict__ gate,
+                                                         bf16* __restrict__ y, int D, int H, int W, int relu) {
+  static_assert(CIN % 16 == 0 && COUT % (16 * NT) == 0, "channel counts");
+  constexpr int HX = kConvX + 2, HY = kConvY + 2, HV = HX * HY * (ZT + 2);
+  constexpr int CH = CIN / 16, NC = COUT / 16, FR = kConvIters * NT;  // chunks, channel blocks, operands per chunk
+  constexpr bool RES = conv_resident<CIN, NT>();
+  using Loader = HaloLoader<CIN, HX, HY, ZT + 2, WIDE>;
+  constexpr int XU = Loader::XU, WU = (FR * 64 + kConvThreads - 1) / kConvThreads;
+  __shared__ __attribute__((aligned(16))) bf16 tile[2 * HV * 8];
+  __shared__ __attribute__((aligned(16))) bf16 wl[(RES ? CH : 1) * FR * 512];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4, nt0 = blockIdx.y * NT;
+  const int parts = gridDim.x, b = blockIdx.x;
+  const int part = parts % HFSI_NXCD == 0 ? (b % HFSI_NXCD) * (parts / HFSI_NXCD) + b / HFSI_NXCD : b;
+  const int gx = (W + kConvX - 1) / kConvX, gz = (D + ZT - 1) / ZT;
+  const long tiles = conv_row_tiles(D, H, W, ZT);
+  const int tbeg = (int)(tiles * part / parts), tend = (int)(tiles * (part + 1) / parts);
+  if (tbeg >= tend) return;  // the whole workgroup, before any barrier
+  int x0 = tbeg / gz % gx * kConvX, y0 = tbeg / gz / gx * kConvY, z0 = tbeg % gz * ZT;
+  int nx0 = x0, ny0 = y0, nz0 = z0;  // the tile whose input is being loaded
+  // 16-byte unit `unit` (operand unit / 64, lane unit % 64) of this workgroup's channel blocks in a
+  // chunk's packed weights
+  auto packed = [&](int unit) -> uint32_t {
+    return (uint32_t)((unit >> 6) / NT * NC + nt0 + (unit >> 6) % NT) * 512 + (unit & 63) * 8;
+  };
+  constexpr int kChunkWeights = kConvIters * NC * 512;
+  uint32_t woff[RES ? 1 : WU];
+  if (!RES) {
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int cb = 0; cb < CIN; cb += CC) {
-    if (cb) __syncthreads();  // the chunk before is consumed
-    for (int p = tid; p < kConvHaloVox * UNITS; p += kConvThreads) {
-      const int v = p / UNITS, q = p % UNITS;
-      const int hx = v % kConvHaloX, hy = (v / kConvHaloX) % kConvHaloY, hz = v / (kConvHaloX * kConvHaloY);
-      const int gx = tx0 + hx, gy = ty0 + hy, gz = tz0 + hz;
-      bf16x8 val = bf16x8_zero();
-      if (gx >= 0 && gx < W && gy >= 0 && gy < H && gz >= 0 && gz < D)
-        val = *reinterpret_cast<const bf16x8*>(x + (((long)gz * H + gy) * W + gx) * CIN + cb + 8 * q);
-      *reinterpret_cast<bf16x8*>(tile + v * VS + 8 * q) = val;
-    }
-    __syncthreads();
-    // the weight operand of K block it comes from global memory (L2): loaded PD blocks ahead of its
-    // use into a ring of registers, so that the MFMAs do not wait on each load in turn
-    auto load_b = [&](int it, bf16x8 (&b)[NT]) {
-      const int u = 4 * it + g;
-      const bool ok = u < KU;
-      const int tap = ok ? u / UNITS : 0, cu = ok ? u % UNITS : 0;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-        b[nt] = ok ? *reinterpret_cast<const bf16x8*>(wt + (size_t)(nt * 16 + r) * KP + tap * CIN + cb + 8 * cu)
-                   : bf16x8_zero();
-    };
-    bf16x8 bq[PD + 1][NT];
-#pragma unroll
-    for (int it = 0; it < PD && it < NIT; ++it) load_b(it, bq[it]);
-#pragma unroll
-    for (int it = 0; it < NIT; ++it) {
-      if (it + PD < NIT) load_b(it + PD, bq[(it + PD) % (PD + 1)]);
-      const int u = 4 * it + g;
-      const bool ok = u < KU;
-      const int tap = ok ? u / UNITS : 0, cu = ok ? u % UNITS : 0;
-      int dz, dy, dx;
-      tap_offset(tap, dz, dy, dx);
-      const bf16* a0 = tile + ((1 + dz) * kConvHaloY * kConvHaloX + (ly + dy) * kConvHaloX + (lx + dx)) * VS + 8 * cu;
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const bf16x8 a = ok ? *reinterpret_cast<const bf16x8*>(a0 + mt * kConvHaloY * kConvHaloX * VS) : bf16x8_zero();
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bq[it % (PD + 1)][nt], acc[mt][nt], 0, 0, 0);
-      }
-    }
+    for (int q = 0; q < WU; ++q) woff[q] = packed(tid + q * kConvThreads);
   }
-  // Output through LDS, 16 output channels at a time: each wave writes its 64 voxels x 16 channels
-  // (bf16, bias and activation applied) into its own 2 KB of the finished tile, then every lane
-  // stores two 16-byte runs of 8 channels of one voxel (rather than 16 two-byte stores of one
-  // channel each).  Every wave takes part in the barriers; voxels outside the grid are skipped at
-  // the store.
-  static_assert(kConvHaloVox * VS >= 4 * 64 * 16, "the output staging fits the input tile");
-  bf16* stage = tile + wave * 64 * 16;
+  Loader loader;
+  loader.init(H, W);
+  bf16x8 rx[XU], rw[RES ? 1 : WU];
+  auto load = [&](int c) {
+    loader.load(in, 16 * c, nx0, ny0, nz0, D, H, W, rx);
+    if (!RES) {
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    __syncthreads();  // the tile (or the previous channel block's staging) is no longer read
-    const int co = nt * 16 + r;
-    const float bv = bias ? bias[co] : 0.0f;
+      for (int q = 0; q < WU; ++q)
+        if (tid + q * kConvThreads < FR * 64)
+          rw[q] = *reinterpret_cast<const bf16x8*>(wt + c * kChunkWeights + woff[q]);
+    }
+  };
+  load(0);
+  if (RES)
+    for (int c = 0; c < CH; ++c)
+      for (int u = tid; u < FR * 64; u += kConvThreads)
+        *reinterpret_cast<bf16x8*>(wl + (c * FR * 64 + u) * 8) =
+            *reinterpret_cast<const bf16x8*>(wt + c * kChunkWeights + packed(u));
+  f32x4 bv[NT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+  for (int nt = 0; nt < NT; ++nt)
+    bv[nt] = bias ? *reinterpret_cast<const f32x4_u*>(bias + (nt0 + nt) * 16 + 4 * g) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // this lane's voxel of the wave's first row at the tap and plane of each MFMA
+  const int row0 = wave * ZT;  // row rr of the tile: y = rr % 4, z = rr / 4
+  int off[kConvIters];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float o = acc[mt][nt][i] + bv;
-        if (RELU) o = fmaxf(o, 0.0f);
-        stage[(mt * 16 + 4 * g + i) * 16 + r] = (bf16)o;  // voxel (i, g) of z-slice mt, channel r
+  for (int it = 0; it < kConvIters; ++it) {
+    const int u = min(4 * it + g, kConvUnits - 1), tap = u >> 1;
+    off[it] = ((u & 1) * HV + (tap / 9 * HY + tap / 3 % 3) * HX + tap % 3 + r) * 8;
+  }
+  const bool pad = 4 * (kConvIters - 1) + g >= kConvUnits;  // this lane's units of the last MFMA
+  const uint32_t lane_out = r * COUT + nt0 * 16 + 4 * g;
+  // what `load` fetched, into LDS
+  auto put = [&] {
+#pragma unroll
+    for (int q = 0; q < XU; ++q) {
+      const int p = tid + q * kConvThreads;
+      if (p < 2 * HV) *reinterpret_cast<bf16x8*>(tile + ((p & 1) * HV + (p >> 1)) * 8) = rx[q];
+    }
+    if (!RES) {
+#pragma unroll
+      for (int q = 0; q < WU; ++q)
+        if (tid + q * kConvThreads < FR * 64) *reinterpret_cast<bf16x8*>(wl + (tid + q * kConvThreads) * 8) = rw[q];
+    }
+  };
+  put();
+  __syncthreads();
+  f32x4 acc[ZT][NT];
+  for (int t = tbeg; t < tend; ++t) {
+#pragma unroll
+    for (int m = 0; m < ZT; ++m)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[m][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c = 0; c < CH; ++c) {
+      const bool more = c + 1 < CH || t + 1 < tend;
+      if (c + 1 < CH) {
+        load(c + 1);
+      } else if (more) {
+        next_tile<kConvX, kConvY, ZT>(nx0, ny0, nz0, D, W);
+        load(0);
       }
-    __syncthreads();
+      const bf16* w0 = wl + (RES ? c * FR * 512 : 0) + lane * 8;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int q = lane;  // voxel of the wave's brick: z-slice q / 16, row q % 16 = 4 g' + i'
-      const int ox = bx0 + (q & 3), oy = by0 + ((q >> 2) & 3), oz = bz0 + (q >> 4);
-      bf16x8 v8 = *reinterpret_cast<const bf16x8*>(stage + q * 16 + 8 * h);
-      if (ox < W && oy < H && oz < D) {
-        const long v = ((long)oz * H + oy) * W + ox;
-        if (gate) v8 = relu_gate(v8, *reinterpret_cast<const bf16x8*>(gate + v * ycs + yoff + nt * 16 + 8 * h));
-        *reinterpret_cast<bf16x8*>(y + v * ycs + yoff + nt * 16 + 8 * h) = v8;
+      for (int it = 0; it < kConvIters; ++it) {
+        bf16x8 a[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) a[nt] = *reinterpret_cast<const bf16x8*>(w0 + (it * NT + nt) * 512);
+        const bf16* b0 = tile + off[it] + ((row0 >> 2) * HY + (row0 & 3)) * HX * 8;
+#pragma unroll
+        for (int m = 0; m < ZT; ++m) {  // rows row0 .. row0 + ZT - 1 lie in one z-slice
+          bf16x8 v = *reinterpret_cast<const bf16x8*>(b0 + m * HX * 8);
+          if (it == kConvIters - 1 && pad) v = bf16x8_zero();
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt)
+            acc[m][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[nt], v, acc[m][nt], 0, 0, 0);
+        }
+      }
+      if (c + 1 < CH) {
+        __syncthreads();  // consumed
+        put();
+        __syncthreads();
       }
     }
+    __syncthreads();  // the tile is consumed
+    // before this tile's stores are issued: its loads are older, and waiting for them then does not wait
+    // for the stores
+    if (t + 1 < tend) put();
+    const bool in_x = x0 + r < W;
+#pragma unroll
+    for (int m = 0; m < ZT; ++m) {
+      const int rr = row0 + m, oy = y0 + (rr & 3), oz = z0 + (rr >> 2);
+      if (oy >= H || oz >= D) continue;  // the whole wave
+      const long row = (((long)oz * H + oy) * W + x0) * COUT;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        bf16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float s = acc[m][nt][e] + bv[nt][e];
+          if (relu) s = fmaxf(s, 0.0f);
+          o[e] = (bf16)s;
+        }
+        if (gate && in_x) {
+          const bf16x4 act = *reinterpret_cast<const bf16x4*>(gate + row + lane_out + nt * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (!((float)act[e] > 0.0f)) o[e] = (bf16)0.0f;
+        }
+        if (in_x) *reinterpret_cast<bf16x4*>(y + row + lane_out + nt * 16) = o;
+      }
+    }
+    next_tile<kConvX, kConvY, ZT>(x0, y0, z0, D, W);
+    __syncthreads();
   }
 }
 
@@ -233,9 +369,16 @@ __global__ void __launch_bounds__(kConvThreads) k_conv3_fwd(const bf16* __restri
 // 16 x 16 gradient took 69 us at 64^3 and the 48 x 16 one 227 us, and a bias pass 67 us more; now
 // 17.8 and 47.9 us with the bias.
 constexpr int kWgTaps = 28, kWgWaveTaps = 7;
+constexpr int kConvTileX = 8, kConvTileY = 8, kConvTileZ = 4;
 constexpr int kWgVox = kConvTileX * kConvTileY * kConvTileZ;  // 256
+constexpr int kConvHaloX = kConvTileX + 2, kConvHaloY = kConvTileY + 2, kConvHaloZ = kConvTileZ + 2;
+constexpr int kConvHaloVox = kConvHaloX * kConvHaloY * kConvHaloZ;  // 600
 
-typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
+__host__ __device__ inline int conv_tiles(int D, int H, int W) {
+  return ((W + kConvTileX - 1) / kConvTileX) * ((H + kConvTileY - 1) / kConvTileY) *
+         ((D + kConvTileZ - 1) / kConvTileZ);
+}
+
 typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
 
 // Channel (lane % 16) of the 8 voxels p, p + 16, .. p + 112 bf16 (x neighbours of one row).
@@ -254,12 +397,13 @@ __host__ __device__ inline int wgrad_parts(int tiles, int cin) {
   return n / HFSI_NXCD * HFSI_NXCD;
 }
 
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(kConvThreads) k_conv3_wgrad(const bf16* __restrict__ x, const bf16* __restrict__ dy,
+template <int CIN, int COUT, bool WIDE>
+__global__ void __launch_bounds__(kConvThreads) k_conv3_wgrad(ConvIn in, const bf16* __restrict__ dy,
                                                                float* __restrict__ partial, int D, int H, int W) {
   static_assert(CIN % 16 == 0 && COUT % 16 == 0, "channel counts");
   constexpr int MT = COUT / 16;
-  constexpr int XU = (kConvHaloVox * 2 + kConvThreads - 1) / kConvThreads;  // 16-byte units per thread
+  using Loader = HaloLoader<CIN, kConvHaloX, kConvHaloY, kConvHaloZ, WIDE>;
+  constexpr int XU = Loader::XU;  // 16-byte units per thread
   constexpr int YU = kWgVox * (COUT / 8) / kConvThreads;
   __shared__ __attribute__((aligned(16))) bf16 sx[kConvHaloVox * 16];
   __shared__ __attribute__((aligned(16))) bf16 sdy[MT * kWgVox * 16];
@@ -270,37 +414,45 @@ __global__ void __launch_bounds__(kConvThreads) k_conv3_wgrad(const bf16* __rest
   const int gx = (W + kConvTileX - 1) / kConvTileX, gz = (D + kConvTileZ - 1) / kConvTileZ;
   const long tiles = conv_tiles(D, H, W);
   const int tbeg = (int)(tiles * part / parts), tend = (int)(tiles * (part + 1) / parts);
+  int x0 = tbeg / gz % gx * kConvTileX, y0 = tbeg / gz / gx * kConvTileY, z0 = tbeg % gz * kConvTileZ;
+  Loader loader;
+  loader.init(H, W);
+  uint32_t yoff[YU];  // this thread's dy units, from the tile's corner
+#pragma unroll
+  for (int q = 0; q < YU; ++q) {
+    const uint32_t p = tid + q * kConvThreads, v = p / (COUT / 8), u = p % (COUT / 8);
+    yoff[q] = (((v >> 6) * H + (v >> 3 & 7)) * W + (v & 7)) * (COUT * 2) + 16 * u;
+  }
   f32x4 acc[kWgWaveTaps][MT];
 #pragma unroll
   for (int j = 0; j < kWgWaveTaps; ++j)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[j][mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   bf16x8 rx[XU], ry[YU];
-  auto load = [&](int t) {
-    const int column = t / gz;
-    const int x0 = (column % gx) * kConvTileX, y0 = (column / gx) * kConvTileY, z0 = (t % gz) * kConvTileZ;
-#pragma unroll
-    for (int q = 0; q < XU; ++q) {
-      const int p = tid + q * kConvThreads, v = p >> 1;
-      const int xx = x0 - 1 + v % kConvHaloX, yy = y0 - 1 + (v / kConvHaloX) % kConvHaloY,
-                zz = z0 - 1 + v / (kConvHaloX * kConvHaloY);
-      rx[q] = bf16x8_zero();
-      if (v < kConvHaloVox && xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D)
-        rx[q] = *reinterpret_cast<const bf16x8*>(x + (((long)zz * H + yy) * W + xx) * CIN + cb + 8 * (p & 1));
-    }
+  auto load = [&] {
+    loader.load(in, cb, x0, y0, z0, D, H, W, rx);
+    const bf16* corner = dy + (((long)z0 * H + y0) * W + x0) * COUT;
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(corner), 0, (int)(uint32_t)kConvSpan, 0x00027000);
+    const bool inner = x0 + kConvTileX <= W && y0 + kConvTileY <= H && z0 + kConvTileZ <= D;
 #pragma unroll
     for (int q = 0; q < YU; ++q) {
-      const int p = tid + q * kConvThreads, v = p / (COUT / 8), u = p % (COUT / 8);
-      const int xx = x0 + (v & 7), yy = y0 + ((v >> 3) & 7), zz = z0 + (v >> 6);
-      ry[q] = bf16x8_zero();
-      if (xx < W && yy < H && zz < D)
-        ry[q] = *reinterpret_cast<const bf16x8*>(dy + (((long)zz * H + yy) * W + xx) * COUT + 8 * u);
+      const int v = (tid + q * kConvThreads) / (COUT / 8);
+      const bool valid = inner || (x0 + (v & 7) < W && y0 + (v >> 3 & 7) < H && z0 + (v >> 6) < D);
+      if constexpr (!WIDE) {
+        ry[q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(valid ? yoff[q] : ~0u), 0, 0));
+      } else {
+        ry[q] = bf16x8_zero();
+        if (valid)
+          ry[q] = *reinterpret_cast<const bf16x8*>(corner + (((long)(v >> 6) * H + (v >> 3 & 7)) * W + (v & 7)) * COUT +
+                                                   8 * ((tid + q * kConvThreads) % (COUT / 8)));
+      }
     }
+    next_tile<kConvTileX, kConvTileY, kConvTileZ>(x0, y0, z0, D, W);
   };
   bf16x8 ones;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = (bf16)1.0f;
-  if (tbeg < tend) load(tbeg);
+  if (tbeg < tend) load();
   for (int t = tbeg; t < tend; ++t) {
     __syncthreads();  // the tile before is consumed
 #pragma unroll
@@ -314,7 +466,7 @@ __global__ void __launch_bounds__(kConvThreads) k_conv3_wgrad(const bf16* __rest
       *reinterpret_cast<bf16x8*>(sdy + ((u >> 1) * kWgVox + v) * 16 + 8 * (u & 1)) = ry[q];
     }
     __syncthreads();
-    if (t + 1 < tend) load(t + 1);
+    if (t + 1 < tend) load();
 #pragma unroll 2
     for (int kb = 0; kb < kWgVox / 32; ++kb) {
       const int z = kb >> 1, y = 4 * (kb & 1) + g, xv = i >> 2, c = 4 * (i & 3);
@@ -432,27 +584,6 @@ __global__ void k_skip_pool_bwd(const bf16* __restrict__ dout, const bf16* __res
   }
 }
 
-// out[v][0:CC] = coarse[parent(v)], out[v][CC:CC+CS] = skip[v]   (fine dims D, H, W)
-__global__ void k_upcat_fwd(const bf16* __restrict__ coarse, const bf16* __restrict__ skip, bf16* __restrict__ out,
-                            int D, int H, int W, int CC, int CS) {
-  // one thread per 8-channel unit of an output voxel (CC and CS are multiples of 8): 16-byte copies
-  const int UC = CC / 8, U = (CC + CS) / 8, C = CC + CS;
-  const long n = (long)D * H * W * U;
-  const int hh = H / 2, w = W / 2;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int u = (int)(i % U);
-    const long v = i / U;
-    bf16x8 val;
-    if (u < UC) {
-      const int X = (int)(v % W), Y = (int)((v / W) % H), Z = (int)(v / ((long)W * H));
-      val = *reinterpret_cast<const bf16x8*>(coarse + ((((long)(Z / 2) * hh) + Y / 2) * w + X / 2) * CC + 8 * u);
-    } else {
-      val = *reinterpret_cast<const bf16x8*>(skip + v * CS + 8 * (u - UC));
-    }
-    *reinterpret_cast<bf16x8*>(out + v * C + 8 * u) = val;
-  }
-}
-
 // dcoarse[p][c] = sum of the 8 children's dout[v][c] (c < CC) through the ReLU of the coarse output y.
 __global__ void k_upcat_bwd_coarse(const bf16* __restrict__ dout, const bf16* __restrict__ y,
                                    bf16* __restrict__ dcoarse, int D, int H, int W, int CC, int CS) {
@@ -552,30 +683,26 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
   }
 }
 
-// bf16 working weights of every conv layer from its float32 master [cout][27 cin]:
-// forward [cout][KP(cin)] and flipped-transposed [cin][KP(cout)], zero padded.
+// bf16 working weights of every conv layer from its float32 master [cout][27 cin], packed as k_conv3
+// reads them: forward (wf), and for the data gradient with taps flipped and channels swapped (wb).
 constexpr int kWeightsPerBlock = 1024;
 __global__ void __launch_bounds__(256) k_conv_weights(ConvLayers tab, const float* __restrict__ params) {
   const ConvLayer& L = tab.l[conv_layer_of(tab, blockIdx.x)];
   const float* wm = params + L.w_off;
-  const int cin = L.cin, cout = L.cout;
-  const int kpf = conv_kp(cin), kpb = conv_kp(cout);
-  const int nf = cout * kpf, nb = L.wb ? cin * kpb : 0;
+  const int nf = conv_packed(L.cin, L.cout), nb = L.wb ? conv_packed(L.cout, L.cin) : 0;
   const int base = (blockIdx.x - L.first) * kWeightsPerBlock;
   for (int i = base + threadIdx.x; i < min(nf + nb, base + kWeightsPerBlock); i += blockDim.x) {
-    if (i < nf) {
-      const int co = i / kpf, k = i % kpf;
-      L.wf[i] = (bf16)(k < 27 * cin ? wm[(size_t)co * 27 * cin + k] : 0.0f);
-    } else {
-      const int j = i - nf;
-      const int ci = j / kpb, k = j % kpb;
-      float val = 0.0f;
-      if (k < 27 * cout) {
-        const int tapb = k / cout, co = k % cout;
-        val = wm[(size_t)co * 27 * cin + (26 - tapb) * cin + ci];
-      }
-      L.wb[j] = (bf16)val;
-    }
+    const bool back = i >= nf;
+    const int j = back ? i - nf : i;
+    const int nc = (back ? L.cin : L.cout) / 16;  // output channel blocks
+    const int e = j & 7, l = j >> 3 & 63, f = j >> 9;
+    const int nt = f % nc, it = f / nc % kConvIters, c = f / nc / kConvIters;
+    const int u = 4 * it + (l >> 4);
+    const int co = 16 * nt + (l & 15), ci = 16 * c + 8 * (u & 1) + e, tap = u >> 1;
+    float val = 0.0f;
+    if (u < kConvUnits)
+      val = back ? wm[(size_t)ci * 27 * L.cin + (26 - tap) * L.cin + co] : wm[(size_t)co * 27 * L.cin + tap * L.cin + ci];
+    (back ? L.wb : L.wf)[j] = (bf16)val;
   }
 }
 

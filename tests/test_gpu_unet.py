@@ -262,8 +262,13 @@ def test_adam_first_step_closed_form_and_training_reduces_loss():
 def test_gradients_at_tile_edges(shape):
     """Weight and bias gradients where the 8 x 8 x 4 voxel tiles are cut by the grid on one, two or three
     axes and where there are fewer tiles than XCDs, and their accumulation over two backward passes
-    (twice the single gradient, exactly: the sums are deterministic).  Tolerance as in
-    test_gradients_match_cpu_autograd."""
+    (twice the single gradient, exactly: the sums are deterministic).
+
+    Tolerance: 3e-2 as in test_gradients_match_cpu_autograd, plus the distance between the CPU gradients
+    with and without bf16 storage.  A sum that lands on the other side of a bf16 rounding boundary early
+    in the network changes the roundings (and the open ReLUs) of all that follow, up to the level of the
+    bf16 rounding itself, which is that distance (measured 0.02 to 0.09 per layer); a wrong tap, edge or
+    tile gives differences of order one."""
     _say(f"unet gradients at {shape}")
     _lib, L, h, params, stream = _setup(shape, 21)
     x5 = _inputs(shape, 22)
@@ -282,15 +287,18 @@ def test_gradients_at_tile_edges(shape):
     np.testing.assert_array_equal(grads[1], np.float32(2.0) * grads[0])
     x = torch.zeros((1, 16) + shape, dtype=torch.float64)
     x[0, :5] = _bf16(x5).permute(3, 0, 1, 2)
-    cp = _cpu_params(params, grad=True)
-    (_cpu_net(cp, x)[0] * torch.from_numpy(dy.astype(np.float64))).sum().backward()
+    ref = []
+    for storage in (True, False):
+        cp = _cpu_params(params, grad=True)
+        (_cpu_net(cp, x, bf16_storage=storage)[0] * torch.from_numpy(dy.astype(np.float64))).sum().backward()
+        ref.append({k: tuple(t.grad.numpy() for t in v) for k, v in cp.items()})
     gsplit = _split(grads[0].astype(np.float64))
     for name, cin, cout in LAYERS + [("OUT", 16, 1)]:
-        for got, ref in zip(gsplit[name], cp[name]):
-            ref = ref.grad.numpy()
+        for got, want, unrounded in zip(gsplit[name], ref[0][name], ref[1][name]):
             if name == "E1A" and got.ndim == 5:
-                got, ref = got[:, :5], ref[:, :5]
-            err = np.linalg.norm(got - ref) / max(np.linalg.norm(ref), 1e-30)
-            _say(f"  {name} {got.shape}: {err:.2e}")
-            assert err < 3e-2, (name, err)
+                got, want, unrounded = got[:, :5], want[:, :5], unrounded[:, :5]
+            scale = max(np.linalg.norm(want), 1e-30)
+            err, noise = np.linalg.norm(got - want) / scale, np.linalg.norm(unrounded - want) / scale
+            _say(f"  {name} {got.shape}: {err:.2e} (bf16 storage: {noise:.2e})")
+            assert err < 3e-2 + noise, (name, err, noise)
     L.hfsi_unet_destroy(h)
