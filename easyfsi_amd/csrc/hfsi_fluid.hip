@@ -1346,10 +1346,12 @@ struct TailLevel {
   TV* rhs;
 };
 
-// LDS layout of the tail levels (byte offsets into dynamic shared memory).
+// LDS layout of the tail levels (byte offsets into dynamic shared memory).  The flags, coefficients and
+// widths of all levels form one image, packed in global memory when the masks are set (k_tail_pack).
 struct TailLdsPlan {
   uint32_t bytes;  // 0: the tail does not fit, run it from global memory
-  uint32_t off_lv;
+  uint32_t off_image, image_bytes;
+  uint32_t off_work;  // C per cell of the largest level that is prolongated onto
   uint32_t off_p[kMaxLevels], off_t[kMaxLevels], off_rhs[kMaxLevels], off_flags[kMaxLevels];
   uint32_t off_cl[kMaxLevels][3], off_ch[kMaxLevels][3], off_wf[kMaxLevels][3];
 };
@@ -1449,43 +1451,291 @@ __device__ inline void block_copy(T* dst, const T* src, uint32_t n) {
   for (uint32_t c = threadIdx.x; c < n; c += blockDim.x) dst[c] = src[c];
 }
 
-// Same V-cycle tail with every level's iterates, masks and coefficients in LDS.
+// The image of the tail's flags and metrics, laid out as the tail workgroup holds it in LDS.
 template <typename C>
-__global__ void __launch_bounds__(kTailThreads) k_vcycle_tail_lds(const TailArgs<C, float>* args, int pre,
-                                                                  int coarse, int post, C omega, C scale) {
-  extern __shared__ __align__(16) unsigned char smem[];
+__global__ void __launch_bounds__(kTailThreads) k_tail_pack(const TailArgs<C, float>* args, unsigned char* image) {
   const TailArgs<C, float>& A = *args;
   const TailLdsPlan& P = A.plan;
-  TailLevel<C, float>* lv = reinterpret_cast<TailLevel<C, float>*>(smem + P.off_lv);
-  const int first = A.first, last = A.last;
-  if ((int)threadIdx.x >= first && (int)threadIdx.x <= last) {
-    const int l = threadIdx.x;
-    TailLevel<C, float> L = A.lv[l];
-    L.g.flags = smem + P.off_flags[l];
-    for (int a = 0; a < 3; ++a) {
-      L.g.cl[a] = reinterpret_cast<const C*>(smem + P.off_cl[l][a]);
-      L.g.ch[a] = reinterpret_cast<const C*>(smem + P.off_ch[l][a]);
-      L.g.wf[a] = reinterpret_cast<const float*>(smem + P.off_wf[l][a]);
-    }
-    L.p = reinterpret_cast<float*>(smem + P.off_p[l]);
-    L.t = reinterpret_cast<float*>(smem + P.off_t[l]);
-    L.rhs = reinterpret_cast<float*>(smem + P.off_rhs[l]);
-    lv[l] = L;
-  }
-  for (int l = first; l <= last; ++l) {
+  unsigned char* at = image - P.off_image;
+  for (int l = A.first; l <= A.last; ++l) {
     const OpGeo<C>& g = A.lv[l].g;
-    block_copy(smem + P.off_flags[l], g.flags, g.n);
+    block_copy(at + P.off_flags[l], g.flags, g.n);
     const uint32_t len[3] = {g.nx, g.ny, g.nz};
     for (int a = 0; a < 3; ++a) {
-      block_copy(reinterpret_cast<C*>(smem + P.off_cl[l][a]), g.cl[a], len[a]);
-      block_copy(reinterpret_cast<C*>(smem + P.off_ch[l][a]), g.ch[a], len[a]);
-      block_copy(reinterpret_cast<float*>(smem + P.off_wf[l][a]), g.wf[a], len[a]);
+      block_copy(reinterpret_cast<C*>(at + P.off_cl[l][a]), g.cl[a], len[a]);
+      block_copy(reinterpret_cast<C*>(at + P.off_ch[l][a]), g.ch[a], len[a]);
+      block_copy(reinterpret_cast<float*>(at + P.off_wf[l][a]), g.wf[a], len[a]);
     }
   }
+}
+
+// A tail level as the workgroup sees it: LDS byte offsets.
+template <typename C>
+struct TailShape {
+  uint32_t nx, ny, nz, n, sx, sy;
+  uint32_t p, t, rhs, flags, cl[3], ch[3], wf[3];
+  const float* fw;
+  const double* diag;
+  C outlet_add;
+  int outlet;
+};
+
+// The shape of level l in scalar registers.
+template <typename C>
+__device__ inline TailShape<C> tail_shape(const TailShape<C>* shapes, int l) {
+  static_assert(sizeof(TailShape<C>) % 4 == 0, "words");
+  TailShape<C> S;
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(shapes + l);
+  uint32_t* dst = reinterpret_cast<uint32_t*>(&S);
+#pragma unroll
+  for (uint32_t w = 0; w < sizeof(S) / 4; ++w) dst[w] = __builtin_amdgcn_readfirstlane(src[w]);
+  return S;
+}
+
+// The cells of one level that a thread owns (c = base + thread + 1024 q), what does not change between
+// the passes over it: position and open faces, and the diagonal (0 for an obstacle; cells whose diagonal
+// is not positive hold 0).
+constexpr int kTailQ = (int)kTailCells / kTailThreads;
+template <typename C>
+struct TailCells {
+  uint32_t at[kTailQ];  // i | j << 16
+  uint32_t kf[kTailQ];  // k | flags << 16
+  C den[kTailQ];
+};
+
+// c / n for c < 2^20: the quotient's distance to the next integer, 0.5 / n, is far above its error
+__device__ inline uint32_t small_div(uint32_t c, uint32_t n) { return (uint32_t)(((float)c + 0.5f) / (float)n); }
+
+// Neighbour sum (in the order of nb_den) of the cell c at (i, j, k) with flags f, and its diagonal when
+// DEN.  A closed face contributes an exact zero: coefficient 0 times the cell itself.
+template <bool DEN, bool NB, typename C, typename TP>
+__device__ inline void tail_nb(const unsigned char* smem, const TailShape<C>& L, uint32_t c, uint32_t ij, uint32_t kf,
+                               const TP* p, C& nb, C& den) {
+  const uint32_t pos[3] = {ij & 0xffffu, ij >> 16, kf & 0xffffu}, f = kf >> 16;
+  const uint32_t stride[3] = {L.sx, L.sy, 1u};
+  constexpr uint32_t lo_bit[3] = {kXm, kYm, kZm}, hi_bit[3] = {kXp, kYp, kZp};
+  nb = (C)0;
+  den = (C)0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const bool lo = f & lo_bit[a], hi = f & hi_bit[a];
+    C cl = reinterpret_cast<const C*>(smem + L.cl[a])[pos[a]], ch = reinterpret_cast<const C*>(smem + L.ch[a])[pos[a]];
+    const uint32_t cm = lo ? c - stride[a] : c, cp = hi ? c + stride[a] : c;
+    if (L.fw) {
+      cl *= (C)L.fw[c];
+      ch *= (C)L.fw[cp];
+    }
+    cl = lo ? cl : (C)0;
+    ch = hi ? ch : (C)0;
+    if (NB) {
+      nb += cl * (C)p[cm];
+      nb += ch * (C)p[cp];
+    }
+    if (DEN) {
+      den += cl;
+      den += ch;
+    }
+  }
+}
+
+template <typename C>
+__device__ inline void tail_setup(const unsigned char* smem, const TailShape<C>& L, uint32_t base, TailCells<C>& K) {
+#pragma unroll
+  for (int q = 0; q < kTailQ; ++q) {
+    const uint32_t c = base + threadIdx.x + q * kTailThreads;
+    K.at[q] = K.kf[q] = 0;
+    K.den[q] = (C)0;
+    if (c >= L.n) continue;
+    const uint32_t ij = small_div(c, L.nz), k = c - ij * L.nz, i = small_div(ij, L.ny), j = ij - i * L.ny;
+    const uint32_t f = smem[L.flags + c];
+    K.at[q] = i | j << 16;
+    K.kf[q] = k | f << 16;
+    C nb, den;
+    tail_nb<true, false>(smem, L, c, K.at[q], K.kf[q], (const float*)nullptr, nb, den);
+    if (L.outlet && k == 0) den += L.outlet_add;
+    if (L.diag) den += (C)L.diag[c];
+    if (!(f & kObst)) K.den[q] = den;
+  }
+}
+
+// out = one weighted-Jacobi update of p (ZERO: of the zero iterate).
+template <bool ZERO, typename C, typename TP>
+__device__ inline void tail_jacobi(const unsigned char* smem, const TailShape<C>& L, uint32_t base,
+                                   const TailCells<C>& K, const TP* p, float* out, C omega) {
+  const float* rhs = reinterpret_cast<const float*>(smem + L.rhs);
+#pragma unroll
+  for (int q = 0; q < kTailQ; ++q) {
+    const uint32_t c = base + threadIdx.x + q * kTailThreads;
+    if (c >= L.n) continue;
+    C v = (C)0;
+    if (K.den[q] > (C)0) {
+      C nb, unused;
+      tail_nb<false, !ZERO>(smem, L, c, K.at[q], K.kf[q], p, nb, unused);
+      const C pc = ZERO ? (C)0 : (C)p[c];
+      const C jac = (nb - (C)rhs[c]) / K.den[q];
+      v = pc + omega * (jac - pc);
+    }
+    out[c] = (float)v;
+  }
+}
+
+// Same V-cycle tail with every level in LDS, bound by the latency of its ~50 dependent passes.  A
+// thread's cells keep their position and diagonal in registers over a level's passes, LDS is addressed as LDS (the level-pointer form compiled to flat loads), the residual is
+// formed per fine cell before it is gathered, levels of at most 64 cells run in the first wavefront
+// without barriers, and the masks and metrics arrive as one packed image: 107 -> 52 us per V-cycle at
+// 64^3 in float64 (16^3 cells down), bit for bit the same.
+template <typename C>
+__global__ void __launch_bounds__(kTailThreads) k_vcycle_tail_lds(const TailArgs<C, float>* args,
+                                                                  const unsigned char* image, int pre, int coarse,
+                                                                  int post, C omega, C scale) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ TailShape<C> shapes[kMaxLevels];
+  const TailArgs<C, float>& A = *args;
+  const TailLdsPlan& P = A.plan;
+  const int first = A.first, last = A.last, tid = threadIdx.x;
+  for (uint32_t v = tid; v < P.image_bytes / 16; v += kTailThreads)
+    reinterpret_cast<uint4*>(smem + P.off_image)[v] = reinterpret_cast<const uint4*>(image)[v];
   block_copy(reinterpret_cast<float*>(smem + P.off_rhs[first]), A.lv[first].rhs, A.lv[first].g.n);
+  if (tid >= first && tid <= last) {
+    const int l = tid;
+    const OpGeo<C>& g = A.lv[l].g;
+    TailShape<C> S;
+    S.nx = g.nx; S.ny = g.ny; S.nz = g.nz; S.n = g.n; S.sx = g.sx; S.sy = g.sy;
+    S.p = P.off_p[l]; S.t = P.off_t[l]; S.rhs = P.off_rhs[l]; S.flags = P.off_flags[l];
+    for (int a = 0; a < 3; ++a) {
+      S.cl[a] = P.off_cl[l][a];
+      S.ch[a] = P.off_ch[l][a];
+      S.wf[a] = P.off_wf[l][a];
+    }
+    S.fw = g.fw;
+    S.diag = g.diag;
+    S.outlet_add = g.outlet_add;
+    S.outlet = g.outlet;
+    shapes[l] = S;
+  }
   __syncthreads();
-  tail_body<C, float>(lv, first, last, pre, coarse, post, omega, scale);
-  block_copy(A.lv[first].p, reinterpret_cast<const float*>(smem + P.off_p[first]), A.lv[first].g.n);
+  C* work = reinterpret_cast<C*>(smem + P.off_work);
+  auto buf = [&](uint32_t off) { return reinterpret_cast<float*>(smem + off); };
+  // end of a pass over a level of n cells: one wavefront's LDS accesses are in order by themselves
+  auto sync = [](uint32_t n) {
+    if (n <= 64) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    } else {
+      __syncthreads();
+    }
+  };
+  TailCells<C> K;
+  // one pass of `f(base)` over a level's cells; levels beyond a thread's kTailQ cells set up per pass
+  auto each = [&](const TailShape<C>& L, auto f) {
+    if ((uint32_t)(tid & ~63) >= L.n) return;
+    for (uint32_t base = 0; base < L.n; base += kTailCells) {
+      if (L.n > kTailCells) tail_setup(smem, L, base, K);
+      f(base);
+    }
+  };
+  auto begin = [&](const TailShape<C>& L) {
+    if (L.n <= kTailCells && (uint32_t)(tid & ~63) < L.n) tail_setup(smem, L, 0, K);
+  };
+  // where pass m of W over a level writes: the last one to p
+  auto target = [](const TailShape<C>& L, int W, int m) { return (W - m) % 2 == 0 ? L.p : L.t; };
+  const int W = pre + post;
+  for (int l = first; l < last; ++l) {
+    const TailShape<C> L = tail_shape(shapes, l);
+    begin(L);
+    uint32_t out = target(L, W, 1);
+    each(L, [&](uint32_t base) { tail_jacobi<true>(smem, L, base, K, (const float*)nullptr, buf(out), omega); });
+    sync(L.n);
+    uint32_t in = out;
+    for (int m = 2; m <= pre; ++m) {
+      out = target(L, W, m);
+      each(L, [&](uint32_t base) { tail_jacobi<false>(smem, L, base, K, (const float*)buf(in), buf(out), omega); });
+      sync(L.n);
+      in = out;
+    }
+    // residual of every fine cell into the other buffer, then the volume-weighted means
+    const uint32_t res = in == L.p ? L.t : L.p;
+    each(L, [&](uint32_t base) {
+      const float *p = buf(in), *rhs = buf(L.rhs);
+      float* r = buf(res);
+#pragma unroll
+      for (int q = 0; q < kTailQ; ++q) {
+        const uint32_t c = base + tid + q * kTailThreads;
+        if (c >= L.n || (K.kf[q] >> 16 & kObst)) continue;
+        C nb, den;
+        tail_nb<false, true>(smem, L, c, K.at[q], K.kf[q], p, nb, den);
+        r[c] = (float)((C)rhs[c] - (nb - K.den[q] * (C)p[c]));
+      }
+    });
+    sync(L.n);
+    const TailShape<C> G = tail_shape(shapes, l + 1);
+    for (uint32_t c = tid; c < G.n; c += kTailThreads) {
+      C v = (C)0;
+      if (!(smem[G.flags + c] & kObst)) {
+        const uint32_t ij = small_div(c, G.nz), ck = c - ij * G.nz, ci = small_div(ij, G.ny), cj = ij - ci * G.ny;
+        C rsum = (C)0, vsum = (C)0;
+#pragma unroll
+        for (int o = 0; o < 8; ++o) {
+          const uint32_t fi = 2 * ci + (o >> 2), fj = 2 * cj + (o >> 1 & 1), fk = 2 * ck + (o & 1);
+          if (fi < L.nx && fj < L.ny && fk < L.nz) {
+            const uint32_t fc = fi * L.sx + fj * L.sy + fk;
+            if (!(smem[L.flags + fc] & kObst)) {
+              const C vol = (C)(buf(L.wf[0])[fi] * buf(L.wf[1])[fj] * buf(L.wf[2])[fk]);
+              rsum += (C)buf(res)[fc] * vol;
+              vsum += vol;
+            }
+          }
+        }
+        v = rsum / (vsum > (C)1.0e-30 ? vsum : (C)1.0e-30);
+      }
+      buf(G.rhs)[c] = (float)v;
+    }
+    sync(G.n);  // a level of at most 64 cells was written by the wavefront that continues with it
+  }
+  {  // coarsest
+    const TailShape<C> L = tail_shape(shapes, last);
+    begin(L);
+    uint32_t out = target(L, coarse, 1);
+    each(L, [&](uint32_t base) { tail_jacobi<true>(smem, L, base, K, (const float*)nullptr, buf(out), omega); });
+    sync(L.n);
+    uint32_t in = out;
+    for (int m = 2; m <= coarse; ++m) {
+      out = target(L, coarse, m);
+      each(L, [&](uint32_t base) { tail_jacobi<false>(smem, L, base, K, (const float*)buf(in), buf(out), omega); });
+      sync(L.n);
+      in = out;
+    }
+  }
+  for (int l = last - 1; l >= first; --l) {
+    const TailShape<C> L = tail_shape(shapes, l), G = tail_shape(shapes, l + 1);
+    if (L.n > 64 && G.n <= 64) __syncthreads();  // the first wavefront's levels are done
+    begin(L);
+    // the prolongated iterate, unrounded, then the sweeps
+    const uint32_t fine = target(L, W, max(pre, 1));
+    const uint32_t corr = l + 1 == last ? target(G, coarse, max(coarse, 1)) : target(G, W, max(W, pre + 1));
+    for (uint32_t c = tid; c < L.n; c += kTailThreads) {
+      C v = (C)buf(fine)[c];
+      if (!(smem[L.flags + c] & kNotFree)) {
+        const uint32_t ij = small_div(c, L.nz), k = c - ij * L.nz, i = small_div(ij, L.ny), j = ij - i * L.ny;
+        const uint32_t ci = min(i >> 1, G.nx - 1), cj = min(j >> 1, G.ny - 1), ck = min(k >> 1, G.nz - 1);
+        v += scale * (C)buf(corr)[ci * G.sx + cj * G.sy + ck];
+      }
+      work[c] = v;
+    }
+    sync(L.n);
+    uint32_t out = target(L, W, pre + 1);
+    each(L, [&](uint32_t base) { tail_jacobi<false>(smem, L, base, K, (const C*)work, buf(out), omega); });
+    sync(L.n);
+    uint32_t in = out;
+    for (int m = pre + 2; m <= W; ++m) {
+      out = target(L, W, m);
+      each(L, [&](uint32_t base) { tail_jacobi<false>(smem, L, base, K, (const float*)buf(in), buf(out), omega); });
+      sync(L.n);
+      in = out;
+    }
+  }
+  if (A.lv[first].g.n <= 64) __syncthreads();
+  block_copy(A.lv[first].p, (const float*)(smem + P.off_p[first]), A.lv[first].g.n);
 }
 
 // ---------------------------------------------------------------------------
@@ -1569,6 +1819,7 @@ struct hfsi_fluid {
   double* host_totals = nullptr;       // pinned
   void* tail_args_d = nullptr;  // TailArgs<double,float>
   void* tail_args_f = nullptr;  // TailArgs<float,float>
+  unsigned char *tail_image_d = nullptr, *tail_image_f = nullptr;  // packed masks and metrics (k_tail_pack)
   uint32_t tail_lds_bytes_d = 0, tail_lds_bytes_f = 0;
   int tail_outlet = -1;  // outlet switch last written into both tail geometries (-1: none yet)
   // mixed-precision V-cycle (HFSI_PREC_MIXED)
@@ -1957,7 +2208,8 @@ static int run_vcycle(hfsi_fluid* h, T0* P0, T0* T0buf, R0 rhs0, bool zero_init,
     const uint32_t lds = dbl ? h->tail_lds_bytes_d : h->tail_lds_bytes_f;
     if (lds > 0)
       hipLaunchKernelGGL((k_vcycle_tail_lds<C>), dim3(1), dim3(kTailThreads), lds, st,
-                         (const TailArgs<C, float>*)args, pre, coarse, post, omega, scale);
+                         (const TailArgs<C, float>*)args, dbl ? h->tail_image_d : h->tail_image_f, pre, coarse, post,
+                         omega, scale);
     else
       hipLaunchKernelGGL((k_vcycle_tail<C, float>), dim3(1), dim3(kTailThreads), 0, st,
                          (const TailArgs<C, float>*)args, pre, coarse, post, omega, scale);
@@ -2645,21 +2897,14 @@ static int write_tail_args(hfsi_fluid* h, void* dst, hipStream_t st) {
     A.lv[l].t = h->lv[l].t;
     A.lv[l].rhs = h->lv[l].rhs;
   }
-  // LDS plan: level descriptors, then per level p / t / rhs / flags and the
-  // per-axis coefficient and width arrays, 16-byte aligned
+  // LDS plan: the image (per level flags and the per-axis coefficient and width arrays), the prolongation
+  // scratch, then per level p / t / rhs, all 16-byte aligned
   {
     auto al = [](uint32_t v) { return (v + 15u) & ~15u; };
     uint32_t off = 0;
-    A.plan.off_lv = off;
-    off = al(off + (uint32_t)sizeof(TailLevel<C, float>) * kMaxLevels);
+    A.plan.off_image = off;
     for (int l = A.first; l <= A.last && l >= 1; ++l) {
       const LevelMem& m = h->lv[l];
-      A.plan.off_p[l] = off;
-      off = al(off + 4 * m.n);
-      A.plan.off_t[l] = off;
-      off = al(off + 4 * m.n);
-      A.plan.off_rhs[l] = off;
-      off = al(off + 4 * m.n);
       A.plan.off_flags[l] = off;
       off = al(off + m.n);
       const uint32_t len[3] = {m.nx, m.ny, m.nz};
@@ -2672,7 +2917,18 @@ static int write_tail_args(hfsi_fluid* h, void* dst, hipStream_t st) {
         off = al(off + 4 * len[a]);
       }
     }
-    A.plan.bytes = (h->L > 1 && off <= kTailLdsMax) ? off : 0;
+    A.plan.image_bytes = off;
+    A.plan.off_work = off;
+    if (A.first < A.last) off = al(off + (uint32_t)sizeof(C) * h->lv[A.first].n);
+    for (int l = A.first; l <= A.last && l >= 1; ++l) {
+      A.plan.off_p[l] = off;
+      off = al(off + 4 * h->lv[l].n);
+      A.plan.off_t[l] = off;
+      off = al(off + 4 * h->lv[l].n);
+      A.plan.off_rhs[l] = off;
+      off = al(off + 4 * h->lv[l].n);
+    }
+    A.plan.bytes = (h->L > 1 && off <= kTailLdsMax && h->lv[A.first].n < 65536) ? off : 0;
   }
   if (std::is_same<C, double>::value)
     h->tail_lds_bytes_d = A.plan.bytes;
@@ -2681,6 +2937,12 @@ static int write_tail_args(hfsi_fluid* h, void* dst, hipStream_t st) {
   // the outlet flag is per solve: the tail reads outlet from lv[].g.outlet,
   // written below for both values by the solve entry (see set_tail_outlet)
   HFSI_CHECK(hipMemcpyAsync(dst, &A, sizeof(A), hipMemcpyHostToDevice, st));
+  if (A.plan.bytes > 0) {
+    unsigned char*& image = std::is_same<C, double>::value ? h->tail_image_d : h->tail_image_f;
+    if (!image) HFSI_TRY(dalloc(h, &image, A.plan.image_bytes));  // the shapes never change
+    hipLaunchKernelGGL(k_tail_pack<C>, dim3(1), dim3(kTailThreads), 0, st, (const TailArgs<C, float>*)dst, image);
+    HFSI_LAUNCH_CHECK();
+  }
   HFSI_CHECK(hipStreamSynchronize(st));
   return HFSI_OK;
 }
