@@ -222,16 +222,58 @@ __global__ void __launch_bounds__(kBlock) k_jacobi(OpGeo<C> g, P p, R rhs, TOut*
   }
 }
 
-// Thread per coarse cell: fine residual + restriction.
+// Restriction of the fine residual, a tile of 2 x 4 x 8 coarse cells per workgroup: every thread forms
+// the residuals of two fine cells (all their loads in one round trip), which the coarse cells' threads
+// then gather from LDS, in the order and rounding of restrict_cell.
+constexpr uint32_t kRestrictI = 2, kRestrictJ = 4, kRestrictK = 8;
+__host__ __device__ inline uint32_t restrict_tiles(uint32_t n, uint32_t t) { return (n + t - 1) / t; }
+
 template <typename TRes, typename C, typename P, typename R, typename TOut>
-__global__ void __launch_bounds__(kBlock) k_resid_restrict(OpGeo<C> fine, P p, R rhs, OpGeo<C> coarse, TOut* out) {
-  HFSI_CELL_LOOP(coarse.n) {
-    uint32_t ci, cj, ck;
-    decompose(c, coarse.ny, coarse.nz, ci, cj, ck);
-    C v = (C)0;
-    if (!(coarse.flags[c] & kObst)) v = restrict_cell<TRes>(fine, ci, cj, ck, p, rhs);
-    out[c] = (TOut)v;
+__global__ void __launch_bounds__(256) k_restrict_tile(OpGeo<C> fine, P p, R rhs, OpGeo<C> coarse, TOut* out) {
+  constexpr uint32_t kFine = 8 * kRestrictI * kRestrictJ * kRestrictK;
+  __shared__ TRes res[kFine];
+  __shared__ uint8_t flag[kFine];  // kObst also for children outside the grid
+  const uint32_t tk = restrict_tiles(coarse.nz, kRestrictK), tj = restrict_tiles(coarse.ny, kRestrictJ);
+  const uint32_t b = blockIdx.x, bk = b % tk, bj = b / tk % tj, bi = b / tk / tj;
+  const uint32_t ci0 = bi * kRestrictI, cj0 = bj * kRestrictJ, ck0 = bk * kRestrictK;
+#pragma unroll
+  for (uint32_t q = 0; q < kFine / 256; ++q) {
+    const uint32_t t = threadIdx.x + 256 * q;
+    const uint32_t i = 2 * ci0 + t / (4 * kRestrictJ * kRestrictK), j = 2 * cj0 + t / (2 * kRestrictK) % (2 * kRestrictJ),
+                   k = 2 * ck0 + t % (2 * kRestrictK);
+    uint8_t f = kObst;
+    TRes v = (TRes)0;
+    if (i < fine.nx && j < fine.ny && k < fine.nz) {
+      const uint32_t c = i * fine.sx + j * fine.sy + k;
+      f = fine.flags[c];
+      v = (TRes)residual_cell(fine, c, i, j, k, p, rhs);
+    }
+    res[t] = v;
+    flag[t] = f;
   }
+  __syncthreads();
+  const uint32_t t = threadIdx.x;
+  if (t >= kRestrictI * kRestrictJ * kRestrictK) return;
+  const uint32_t lk = t % kRestrictK, lj = t / kRestrictK % kRestrictJ, li = t / (kRestrictK * kRestrictJ);
+  const uint32_t ci = ci0 + li, cj = cj0 + lj, ck = ck0 + lk;
+  if (ci >= coarse.nx || cj >= coarse.ny || ck >= coarse.nz) return;
+  const uint32_t c = ci * coarse.sx + cj * coarse.sy + ck;
+  C v = (C)0;
+  if (!(coarse.flags[c] & kObst)) {
+    C rsum = (C)0, vsum = (C)0;
+#pragma unroll
+    for (uint32_t o = 0; o < 8; ++o) {
+      const uint32_t oi = o >> 2, oj = o >> 1 & 1, ok = o & 1;
+      const uint32_t at = ((2 * li + oi) * 2 * kRestrictJ + 2 * lj + oj) * 2 * kRestrictK + 2 * lk + ok;
+      if (!(flag[at] & kObst)) {
+        const C vol = (C)(fine.wf[0][2 * ci + oi] * fine.wf[1][2 * cj + oj] * fine.wf[2][2 * ck + ok]);
+        rsum += (C)res[at] * vol;
+        vsum += vol;
+      }
+    }
+    v = rsum / (vsum > (C)1.0e-30 ? vsum : (C)1.0e-30);
+  }
+  out[c] = (TOut)v;
 }
 
 // q = A d with the per-workgroup partials of <d, q>_V (combined by k_finish_sums).

@@ -35,6 +35,9 @@ void set_error(const std::string& msg) { g_last_error = msg; }
 
 constexpr int kMaxLevels = 16;
 constexpr uint32_t kMaxGrid = 2048;      // workgroups of full-grid launches (8 per CU)
+// Levels at most this big restrict in tiles: float64 64^3 11.4 -> 8.8 us, 32^3 12.6 -> 7.4 us against the
+// marching form, whose columns leave most of the chip idle there; at 128^3 13.9 (marching) against 22.0 us.
+constexpr uint32_t kRestrictTileMax = 1u << 19;
 constexpr uint32_t kTailCells = 4096;    // levels at most this big run in the single-workgroup tail
 // the same for the mixed V-cycle's LDS-resident tail: one workgroup on one CU; a 23^3 level there
 // (12 167 cells, 110 KB of LDS) took longer than its own multi-workgroup passes (103 us against
@@ -2053,6 +2056,18 @@ static void launch_march(hfsi_fluid* h, int l, int outlet, const TP* p, const TR
   if (DOTS) finish_sums<march_sums<MODE>()>(h, march_grid(a.m), fin, st);
 }
 
+// The marching restriction where its columns fill the chip.
+static bool march_restrict_pays(const hfsi_fluid* h, int l) { return march_ok(h, l) && h->lv[l].n > kRestrictTileMax; }
+
+// Tile restriction l -> l + 1 (any grid).
+template <typename TRes, typename C, typename P, typename R>
+static void launch_restrict_tile(hfsi_fluid* h, int l, int outlet, P p, R rhs, hipStream_t st) {
+  const OpGeo<C> c = geo<C>(h, l + 1, outlet);
+  const uint32_t blocks = restrict_tiles(c.nx, kRestrictI) * restrict_tiles(c.ny, kRestrictJ) * restrict_tiles(c.nz, kRestrictK);
+  hipLaunchKernelGGL((k_restrict_tile<TRes, C, P, R, float>), dim3(blocks), dim3(256), 0, st, geo<C>(h, l, outlet), p,
+                     rhs, c, h->lv[l + 1].rhs);
+}
+
 template <typename C, typename TP, typename TR, typename TRes>
 static void launch_march_restrict(hfsi_fluid* h, int l, int outlet, const TP* p, const TR* rhs, C sign,
                                   hipStream_t st) {
@@ -2156,13 +2171,10 @@ static int run_vcycle(hfsi_fluid* h, T0* P0, T0* T0buf, R0 rhs0, bool zero_init,
     in0 = out;
   }
   timer_mark(h, HFSI_TIMER_L0_RESTRICT, st);
-  if (m0) {
+  if (march_restrict_pays(h, 0))
     launch_march_restrict<C, T0, TR0, T0>(h, 0, outlet, in0, rhs0.p, sign0, st);
-  } else {
-    OpGeo<C> g1 = geo<C>(h, 1, outlet);
-    hipLaunchKernelGGL((k_resid_restrict<T0, C, Ld<T0, C>, R0, float>), dim3(blocks_for(g1.n)), dim3(kBlock), 0, st,
-                       g0, Ld<T0, C>{in0}, rhs0, g1, h->lv[1].rhs);
-  }
+  else
+    launch_restrict_tile<T0, C>(h, 0, outlet, Ld<T0, C>{in0}, rhs0, st);
   timer_mark(h, HFSI_TIMER_L0_RESTRICT, st);
   // ---- grid-launched coarse levels down
   float* cur[kMaxLevels] = {};
@@ -2193,13 +2205,10 @@ static int run_vcycle(hfsi_fluid* h, T0* P0, T0* T0buf, R0 rhs0, bool zero_init,
       in = out;
     }
     cur[l] = in;
-    if (mk) {
+    if (march_restrict_pays(h, l))
       launch_march_restrict<C, float, float, float>(h, l, outlet, in, m.rhs, (C)1, st);
-    } else {
-      OpGeo<C> gc = geo<C>(h, l + 1, outlet);
-      hipLaunchKernelGGL((k_resid_restrict<float, C, Ld<float, C>, Ld<float, C>, float>), dim3(blocks_for(gc.n)),
-                         dim3(kBlock), 0, st, g, Ld<float, C>{in}, R, gc, h->lv[l + 1].rhs);
-    }
+    else
+      launch_restrict_tile<float, C>(h, l, outlet, Ld<float, C>{in}, R, st);
   }
   // ---- tail: levels tail .. L-1 in one workgroup
   {
