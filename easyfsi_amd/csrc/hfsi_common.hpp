@@ -63,16 +63,19 @@ struct ChunkRange {
   uint32_t first, end, step;
 };
 
-// Requires gridDim.x to be a multiple of HFSI_NXCD.
-__device__ inline ChunkRange xcd_chunks(uint32_t nchunks) {
+// The chunks of the first `groups` workgroups (a multiple of HFSI_NXCD), for one of them.
+__device__ inline ChunkRange xcd_chunks(uint32_t nchunks, uint32_t groups) {
   const uint32_t b = blockIdx.x;
-  const uint32_t per = gridDim.x / HFSI_NXCD;
+  const uint32_t per = groups / HFSI_NXCD;
   const uint32_t x = b % HFSI_NXCD;
   const uint32_t s = b / HFSI_NXCD;
   const uint32_t lo = (uint32_t)(((uint64_t)nchunks * x) / HFSI_NXCD);
   const uint32_t hi = (uint32_t)(((uint64_t)nchunks * (x + 1)) / HFSI_NXCD);
   return ChunkRange{lo + s, hi, per};
 }
+
+// Requires gridDim.x to be a multiple of HFSI_NXCD.
+__device__ inline ChunkRange xcd_chunks(uint32_t nchunks) { return xcd_chunks(nchunks, gridDim.x); }
 
 // Loop over the cells [0, n) owned by this thread under the XCD-aware chunk
 // decomposition; `c` is the cell index; `continue` moves to the next chunk.

@@ -265,18 +265,16 @@ __device__ inline void mpm_partials(double (&v)[NS], const MpmArgs& a, uint32_t 
   }
 }
 
-// Combine nrows slot-major partial rows and run the finaliser.  The partials come from every XCD,
+// Combine nrows slot-major partial rows.  The partials come from every XCD,
 // so each load misses this XCD's L2: a thread issues the loads of kMpmFinishRows rows (t, t + 512,
 // ...) before adding them in row order, so that up to 2048 rows take one memory round trip; the
 // thread sums are then combined by the workgroup tree (a fixed order).
 constexpr int kMpmFinishThreads = 512;
 constexpr int kMpmFinishRows = 4;
 
-template <int NS, typename Fin>
-__global__ void __launch_bounds__(kMpmFinishThreads) k_mpm_finish(const double* partials, uint32_t nrows,
-                                                                   uint32_t stride, double* totals, Fin fin,
-                                                                   uint64_t maxmask) {
-  __shared__ double lds[NS * (kMpmFinishThreads / 64)];
+template <int NS>
+__device__ inline void finish_rows(const double* partials, uint32_t nrows, uint32_t stride, double* totals,
+                                   uint64_t maxmask, double* lds) {
   double acc[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) acc[s] = ((maxmask >> s) & 1) ? -INFINITY : 0.0;
@@ -298,8 +296,36 @@ __global__ void __launch_bounds__(kMpmFinishThreads) k_mpm_finish(const double* 
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) totals[s] = acc[s];
-    fin(totals);
   }
+}
+
+// One table of partial rows, then the finaliser.
+template <int NS, typename Fin>
+__global__ void __launch_bounds__(kMpmFinishThreads) k_mpm_finish(const double* partials, uint32_t nrows,
+                                                                   uint32_t stride, double* totals, Fin fin,
+                                                                   uint64_t maxmask) {
+  __shared__ double lds[NS * (kMpmFinishThreads / 64)];
+  finish_rows<NS>(partials, nrows, stride, totals, maxmask, lds);
+  if (threadIdx.x == 0) fin(totals);
+}
+
+// Totals 0..40 of a step: the scatter's, the grid update's and the gather's tables, one workgroup
+// each.  A table takes 6 us, nearly all of it latency (one workgroup, two memory round trips), and
+// nothing reads a total before the radial stretch: three launches in the step's chain became one.
+struct StageRows {
+  const double* partials;
+  uint32_t nrows;
+};
+
+__global__ void __launch_bounds__(kMpmFinishThreads) k_mpm_finish_stages(StageRows p2g, StageRows grid, StageRows g2p,
+                                                                          double* totals) {
+  __shared__ double lds[21 * (kMpmFinishThreads / 64)];
+  if (blockIdx.x == 0)
+    finish_rows<12>(p2g.partials, p2g.nrows, p2g.nrows, totals, kP2gMax, lds);
+  else if (blockIdx.x == 1)
+    finish_rows<8>(grid.partials, grid.nrows, grid.nrows, totals + T_TRANS, kGridMax, lds);
+  else
+    finish_rows<21>(g2p.partials, g2p.nrows, g2p.nrows, totals + T_PDISP, 0ull, lds);
 }
 
 __device__ inline void grid_coord(const MpmArgs& a, const float* xp, float X[3]) {
@@ -551,48 +577,69 @@ __global__ void __launch_bounds__(kBlock) k_mpm_p2g(MpmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Cell-binned P2G: particles are bucketed by the 8^3-node block of their
-// stencil base node; one workgroup accumulates a block's particles into a
-// 10^3-node LDS tile with LDS atomics and adds the tile to the grid with one
-// global atomic per touched node value (instead of 27 x 7 per particle).
+// Cell-binned P2G: particles are bucketed by the block of EDGE^3 nodes of their stencil base node; one
+// workgroup sums a block's particles cell by cell into a tile of (EDGE + 2)^3 nodes in LDS, and the
+// grid update gathers every node from the tiles that cover it (or, without tile buffers, the tile is
+// added to the grid with one global atomic per touched node value instead of 27 x 7 per particle).
 // ---------------------------------------------------------------------------
 
-constexpr int kBinEdge = 8;                 // nodes per block edge
-constexpr int kTileEdge = kBinEdge + 2;     // stencil reach of a block
-constexpr int kTileNodes = kTileEdge * kTileEdge * kTileEdge;
+// Blocks of 8^3 nodes have 2.0 tile nodes per cell, and their 512 cells can be ordered by particle
+// count before lanes take them; but a small body has too few of them: 32^3 particles span 27 to 64, and
+// one workgroup's chain of steps sets the time (scatter 66 us, gather 35 us).  Blocks of 4^3 (3.4 tile
+// nodes per cell, a wavefront's lanes are a block's cells) are eight times as many: 12 and 11 us.  The
+// whole step, loaded, with 4^3 against 8^3 blocks (us):
+//   16^3 particles 77 / 89, 32^3 at 4.6 per cell 81 / 163 and at 1.4 80 / 99, 50^3 at 5.2 115 / 244 and at
+//   2.2 118 / 156, 64^3 at 4.6 151 / 229 and at 2.4 168 / 213, 80^3 at 9.0 213 / 370 and at 2.4 236 / 246,
+//   100^3 at 9.0 364 / 535 but at 2.2 442 / 387, 128^3 at 4.6 738 / 707.
+// The line lies where the sparse body's two times meet, by the state's particle capacity (the tile
+// buffers' layout hangs on it).
+constexpr int kFineEdge = 4, kCoarseEdge = 8;
+constexpr int64_t kFineParticles = 1 << 19;
 
-// Components of a block's P2G tile: mass, momentum (3), external force (3).
-constexpr int kTileComps = 7;
-constexpr size_t kTileStride = (size_t)kTileComps * kTileNodes;  // floats per block
-// Blocks up to this many get a tile buffer (28 KB each); larger grids flush tiles with global atomics.
+template <int EDGE>
+struct Tile {
+  static constexpr int kEdge = EDGE + 2;  // stencil reach of a block
+  static constexpr int kNodes = kEdge * kEdge * kEdge;
+  static constexpr int kCells = EDGE * EDGE * EDGE;
+  // components of a block's tile: mass, momentum (3), external force (3)
+  static constexpr size_t kStride = (size_t)7 * kNodes;
+};
+
+// Grids of up to this many blocks of 8^3 nodes get tile buffers (28 KB per 8^3 block, 6 KB per 4^3
+// block, for as many blocks as can hold particles at once: the smaller of the block and the particle
+// count); larger grids flush tiles with global atomics.
 constexpr size_t kMaxTileBlocks = 65536;
+// Grids are taken up to this many blocks of 8^3 nodes (per-block tables of 4 MB each, 32 MB at 4^3).
+constexpr size_t kMaxBlocks = 1u << 20;
 
 struct BinArgs {
+  int32_t edge;            // nodes per block edge: kFineEdge or kCoarseEdge
   int32_t nbx, nby, nbz;   // block grid
   int32_t* key;            // per particle: block, or -1 when out of bounds
   int32_t* rank;           // per particle: slot within its block
   int32_t* count;          // per block
-  int32_t* offset;         // per block: exclusive prefix sum of count
+  int32_t* offset;         // per active block: its first entry of sorted
+  int32_t* slot;           // per active block: its place in the active list
   int32_t* sorted;         // particles ordered by block
   int32_t* cell;           // per in-bounds particle: its stencil base cell within its block
   int32_t* scell;          // cell of each entry of sorted
   int32_t* active;         // blocks with particles (unordered)
   int32_t* nactive;
+  int32_t* nsorted;        // entries of sorted handed out to active blocks
   int32_t* oob;            // out-of-bounds particles (unordered)
   int32_t* noob;
   int32_t* svd;            // particles whose F takes the SVD clamp this step (unordered)
   int32_t* nsvd;
-  int32_t* scan_sums;      // per 1024-block chunk
   // tile path: every active block stores its whole tile (plain stores) and the grid update gathers each
   // node from the (up to 8) tiles that cover it, in a fixed order
-  float* tiles;            // [block][kTileComps][kTileNodes], or nullptr (atomic flush)
+  float* tiles;            // [active block][component][tile node], or nullptr (atomic flush)
   float4* stage;           // per particle: the prepared scatter operands (p2g_stage), 4 float4
   int32_t* need_stamp;     // per block: stamp of the step that last listed it
   int32_t* need_list;      // blocks with nodes a tile covers: the active blocks and their +1 neighbours
   int32_t* nneed;
   int32_t stamp;           // this step's stamp (never 0: need_stamp starts at 0)
   int32_t has_force;       // particles carry an external force (force components stored)
-  int32_t* block_force;    // per block: this step's tile holds force components (some particle has a force)
+  int32_t* block_force;    // per active block: its tile holds force components (some particle has a force)
   int32_t* prev_need;      // the previous step's need list: every grid node outside it is zero
   int32_t* nprev;
   int32_t reset_prev;      // the grid was cleared whole this step: forget the previous list
@@ -603,6 +650,7 @@ __global__ void k_bin_clear(BinArgs b) {
   for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += gridDim.x * blockDim.x) b.count[i] = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     *b.nactive = 0;
+    *b.nsorted = 0;
     *b.noob = 0;
     *b.nsvd = 0;
     if (b.nneed) *b.nneed = 0;
@@ -610,28 +658,81 @@ __global__ void k_bin_clear(BinArgs b) {
   }
 }
 
-// List every block a tile of an active block reaches (the block and its seven +1 neighbours) once: the
-// stamp exchange admits the first marker of a block in this step.
-__global__ void __launch_bounds__(kBlock) k_need_mark(BinArgs b) {
-  const int32_t nact = *b.nactive;
-  for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nact; i += gridDim.x * blockDim.x) {
-    const int32_t k = b.active[i];
-    const int32_t bx = k / (b.nby * b.nbz), by = (k / b.nbz) % b.nby, bz = k % b.nbz;
-    for (int e = 0; e < 8; ++e) {
-      const int32_t x = bx + (e >> 2), y = by + ((e >> 1) & 1), z = bz + (e & 1);
-      if (x >= b.nbx || y >= b.nby || z >= b.nbz) continue;
-      const int32_t k2 = (x * b.nby + y) * b.nbz + z;
-      if (atomicExch(&b.need_stamp[k2], b.stamp) != b.stamp) b.need_list[atomicAdd(b.nneed, 1)] = k2;
+// Lists of the active blocks and of the blocks whose nodes their tiles cover (an active block and its
+// +1 neighbours, so a block is needed when it or one of its seven -1 neighbours is active), and the
+// ranges of `sorted`, one thread per block.  The counts of all eight blocks are loaded at once and a
+// workgroup takes its places in the three lists with one atomic each, so the pass is two memory round
+// trips long at any number of active blocks: 125 blocks of a 64^3-node grid took 7.5 us by marking
+// neighbours from the active list through an exchange each, after two scan launches over the blocks.
+constexpr int kListBlocks = 1024;  // blocks per workgroup: runs of the lists that keep neighbours together
+
+__global__ void __launch_bounds__(kListBlocks) k_bin_lists(BinArgs b) {
+  constexpr int kWaves = kListBlocks / 64;
+  __shared__ int32_t wave_total[3][kWaves], first[3];
+  const int32_t nblk = b.nbx * b.nby * b.nbz;
+  const int32_t k = (int32_t)(blockIdx.x * kListBlocks + threadIdx.x);
+  const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
+  int32_t cnt = 0;
+  bool need = false;
+  if (k < nblk) {
+    cnt = b.count[k];
+    need = cnt > 0;
+    if (b.need_list) {
+      const int32_t bx = k / (b.nby * b.nbz), by = (k / b.nbz) % b.nby, bz = k % b.nbz;
+      int32_t any = 0;
+#pragma unroll
+      for (int e = 1; e < 8; ++e) {
+        const int ex = e >> 2, ey = (e >> 1) & 1, ez = e & 1;
+        const bool in = bx >= ex && by >= ey && bz >= ez;
+        any |= b.count[in ? k - (ex * b.nby + ey) * b.nbz - ez : k];
+      }
+      need = need || any > 0;
     }
+  }
+  const uint64_t below = (1ull << lane) - 1ull;
+  const uint64_t actives = __builtin_amdgcn_ballot_w64(cnt > 0), needs = __builtin_amdgcn_ballot_w64(need);
+  int32_t incl = cnt;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int32_t y = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += y;
+  }
+  if (lane == 63) {
+    wave_total[0][wave] = (int32_t)__builtin_popcountll(actives);
+    wave_total[1][wave] = incl;
+    wave_total[2][wave] = (int32_t)__builtin_popcountll(needs);
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    int32_t sum = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const int32_t t = wave_total[threadIdx.x][w];
+      wave_total[threadIdx.x][w] = sum;
+      sum += t;
+    }
+    int32_t* counter = threadIdx.x == 0 ? b.nactive : threadIdx.x == 1 ? b.nsorted : b.nneed;
+    first[threadIdx.x] = sum > 0 && counter ? atomicAdd(counter, sum) : 0;
+  }
+  __syncthreads();
+  if (cnt > 0) {
+    const int32_t slot = first[0] + wave_total[0][wave] + (int32_t)__builtin_popcountll(actives & below);
+    b.active[slot] = k;
+    b.slot[k] = slot;
+    b.offset[k] = first[1] + wave_total[1][wave] + incl - cnt;
+  }
+  if (need && b.need_list) {
+    b.need_list[first[2] + wave_total[2][wave] + (int32_t)__builtin_popcountll(needs & below)] = k;
+    b.need_stamp[k] = b.stamp;
   }
 }
 
-// Key, rank and list pushes of every particle.  The lanes of a wavefront with the same block take
+// Key and rank of every particle.  The lanes of a wavefront with the same block take
 // their ranks from one atomic (the lowest such lane adds the group's size; every lane adds its
-// position among the group's lanes), and the block's first group pushes the block to the active
-// list; the out-of-bounds lanes of a wavefront reserve their slots of the out-of-bounds list with
+// position among the group's lanes); the out-of-bounds lanes of a wavefront reserve their slots of the out-of-bounds list with
 // one atomic.  The loop over chunks is uniform across the workgroup, so every lane takes part in
 // the ballots.
+template <int EDGE>
 __global__ void __launch_bounds__(kBlock) k_bin_count(MpmArgs a, BinArgs b) {
   const uint32_t n = (uint32_t)a.count;
   const int lane = (int)(threadIdx.x & 63u);
@@ -648,9 +749,9 @@ __global__ void __launch_bounds__(kBlock) k_bin_count(MpmArgs a, BinArgs b) {
       out = stencil_oob(a, X);
       if (!out) {
         const int sx = (int)floorf(X[0] - 0.5f), sy = (int)floorf(X[1] - 0.5f), sz = (int)floorf(X[2] - 0.5f);
-        const int bx = sx / kBinEdge, by = sy / kBinEdge, bz = sz / kBinEdge;
+        const int bx = sx / EDGE, by = sy / EDGE, bz = sz / EDGE;
         k = (bx * b.nby + by) * b.nbz + bz;
-        b.cell[c] = ((sx - bx * kBinEdge) * kBinEdge + (sy - by * kBinEdge)) * kBinEdge + (sz - bz * kBinEdge);
+        b.cell[c] = ((sx - bx * EDGE) * EDGE + (sy - by * EDGE)) * EDGE + (sz - bz * EDGE);
       }
     }
     const uint64_t outs = __builtin_amdgcn_ballot_w64(valid && out);
@@ -677,10 +778,7 @@ __global__ void __launch_bounds__(kBlock) k_bin_count(MpmArgs a, BinArgs b) {
       todo &= ~same;
     }
     int32_t first_rank = 0;
-    if (k >= 0 && lane == leader) {
-      first_rank = atomicAdd(&b.count[k], (int32_t)__builtin_popcountll(group));
-      if (first_rank == 0) b.active[atomicAdd(b.nactive, 1)] = k;
-    }
+    if (k >= 0 && lane == leader) first_rank = atomicAdd(&b.count[k], (int32_t)__builtin_popcountll(group));
     first_rank = __shfl(first_rank, leader, 64);
     const int32_t r = first_rank + (int32_t)__builtin_popcountll(group & below);
     if (valid) {
@@ -688,45 +786,6 @@ __global__ void __launch_bounds__(kBlock) k_bin_count(MpmArgs a, BinArgs b) {
       if (k >= 0) b.rank[c] = r;
     }
   }
-}
-
-// Exclusive prefix sum of count over nb blocks: per-chunk (1024) scan, scan
-// of the chunk sums (<= 1024 chunks, one workgroup), then add.
-constexpr int kScanChunk = 1024;
-
-__global__ void __launch_bounds__(kScanChunk) k_scan_chunks(const int32_t* in, int32_t* out, int32_t n,
-                                                            int32_t* sums) {
-  __shared__ int32_t t[kScanChunk];
-  const int32_t i = blockIdx.x * kScanChunk + threadIdx.x;
-  const int32_t v = i < n ? in[i] : 0;
-  t[threadIdx.x] = v;
-  __syncthreads();
-  for (int off = 1; off < kScanChunk; off <<= 1) {
-    const int32_t add = threadIdx.x >= (unsigned)off ? t[threadIdx.x - off] : 0;
-    __syncthreads();
-    t[threadIdx.x] += add;
-    __syncthreads();
-  }
-  if (i < n) out[i] = t[threadIdx.x] - v;  // exclusive
-  if (threadIdx.x == kScanChunk - 1) sums[blockIdx.x] = t[threadIdx.x];
-}
-
-__global__ void __launch_bounds__(kScanChunk) k_scan_add(int32_t* out, int32_t n, const int32_t* sums,
-                                                         int32_t nchunks) {
-  __shared__ int32_t t[kScanChunk];
-  // every workgroup scans the (<= 1024) chunk sums itself
-  const int32_t v = (int32_t)threadIdx.x < nchunks ? sums[threadIdx.x] : 0;
-  t[threadIdx.x] = v;
-  __syncthreads();
-  for (int off = 1; off < kScanChunk; off <<= 1) {
-    const int32_t add = threadIdx.x >= (unsigned)off ? t[threadIdx.x - off] : 0;
-    __syncthreads();
-    t[threadIdx.x] += add;
-    __syncthreads();
-  }
-  const int32_t base = blockIdx.x > 0 ? t[blockIdx.x - 1] : 0;
-  const int32_t i = blockIdx.x * kScanChunk + threadIdx.x;
-  if (i < n) out[i] += base;
 }
 
 __global__ void __launch_bounds__(kBlock) k_bin_scatter(int32_t n, BinArgs b) {
@@ -740,7 +799,7 @@ __global__ void __launch_bounds__(kBlock) k_bin_scatter(int32_t n, BinArgs b) {
   }
 }
 
-// Binned P2G scatter of one block, a stencil-base cell at a time (no floating-point atomics).  LDS
+// Binned P2G scatter of one block of 8^3 nodes, a stencil-base cell at a time (no floating-point atomics).  LDS
 // float atomics run at about 1/30 of the rate of integer ones on gfx950 (a probe measured ~190 cycles
 // per wavefront instruction per CU with distinct addresses, against ~6 for u32), so the block's
 // particles are added with plain read-modify-writes instead:
@@ -764,10 +823,10 @@ constexpr int kP2gThreads = 128;
 constexpr int kP2gWaves = kP2gThreads / 64;
 constexpr int kP2gChunk = 1024;                      // particles of a block ordered per pass
 constexpr int kP2gPerThread = kP2gChunk / kP2gThreads;
-constexpr int kBlockCells = kBinEdge * kBinEdge * kBinEdge;
+constexpr int kBlockCells = Tile<kCoarseEdge>::kCells;
 constexpr int kCellsPerThread = kBlockCells / kP2gThreads;
 constexpr int kCountBuckets = 8;                     // cells by particle count: >= 8, 7, ..., 1
-constexpr size_t kP2gTileBytes = (size_t)kP2gWaves * kTileNodes * sizeof(float4);  // dynamic LDS
+constexpr size_t kP2gTileBytes = (size_t)kP2gWaves * Tile<kCoarseEdge>::kNodes * sizeof(float4);  // dynamic LDS
 static_assert(kP2gWaves == 2 && kBlockCells % kP2gThreads == 0, "the cell scan assumes two wavefronts");
 static_assert(kP2gChunk < 65536 && kBlockCells < 65536, "cell ranges and lists are 16-bit");
 
@@ -835,8 +894,42 @@ __device__ inline void load_stage(const float4* stage, int32_t p, float4 (&s)[4]
   for (int i = 0; i < 4; ++i) s[i] = src[i];
 }
 
+// A block's wavefront tiles, summed in wavefront order, to its tile buffer or onto the grid.
+template <int EDGE, int WAVES>
+__device__ inline void flush_tiles(const MpmArgs& a, const BinArgs& b, uint32_t ab, int ox0, int oy0, int oz0,
+                                   const float4* wave_tiles) {
+  constexpr int kNodes = Tile<EDGE>::kNodes, kEdge = Tile<EDGE>::kEdge;
+  const uint32_t sx = (uint32_t)a.ny * a.nz, sy = a.nz;
+  for (int i = threadIdx.x; i < kNodes; i += 64 * WAVES) {
+    float4 v = wave_tiles[i];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) {
+      const float4 u = wave_tiles[w * kNodes + i];
+      v.x += u.x;
+      v.y += u.y;
+      v.z += u.z;
+      v.w += u.w;
+    }
+    if (b.tiles) {
+      float* T = b.tiles + (size_t)ab * Tile<EDGE>::kStride;
+      T[i] = v.x;
+      T[kNodes + i] = v.y;
+      T[2 * kNodes + i] = v.z;
+      T[3 * kNodes + i] = v.w;
+      continue;
+    }
+    const int gx = ox0 + i / (kEdge * kEdge), gy = oy0 + (i / kEdge) % kEdge, gz = oz0 + i % kEdge;
+    if (gx >= a.nx || gy >= a.ny || gz >= a.nz) continue;
+    const uint32_t node = (uint32_t)gx * sx + (uint32_t)gy * sy + (uint32_t)gz;
+    if (v.x != 0.0f) atomicAdd(&a.gm[node], v.x);
+    if (v.y != 0.0f) atomicAdd(&a.gv[3 * (size_t)node + 0], v.y);
+    if (v.z != 0.0f) atomicAdd(&a.gv[3 * (size_t)node + 1], v.z);
+    if (v.w != 0.0f) atomicAdd(&a.gv[3 * (size_t)node + 2], v.w);
+  }
+}
+
 __global__ void __launch_bounds__(kP2gThreads, 2) k_mpm_p2g_cells(MpmArgs a, BinArgs b) {
-  extern __shared__ float4 wave_tiles[];  // [kP2gWaves][kTileNodes]: mass, momentum
+  extern __shared__ float4 wave_tiles[];  // [kP2gWaves][Tile<kCoarseEdge>::kNodes]: mass, momentum
   __shared__ uint32_t cell_count[kBlockCells];
   __shared__ uint16_t cell_start[kBlockCells];  // first entry of each cell in order
   __shared__ uint16_t cell_list[kBlockCells];   // occupied cells, largest count first
@@ -845,13 +938,13 @@ __global__ void __launch_bounds__(kP2gThreads, 2) k_mpm_p2g_cells(MpmArgs a, Bin
   __shared__ uint32_t wave0_total;
   __shared__ int32_t order[kP2gChunk];          // the chunk's particles by cell
   const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63u);
-  float4* tile = wave_tiles + (size_t)wave * kTileNodes;
-  const int32_t nact = *b.nactive;
-  for (int32_t ab = blockIdx.x; ab < nact; ab += gridDim.x) {
+  float4* tile = wave_tiles + (size_t)wave * Tile<kCoarseEdge>::kNodes;
+  const ChunkRange cr = xcd_chunks((uint32_t)*b.nactive);
+  for (uint32_t ab = cr.first; ab < cr.end; ab += cr.step) {
     const int32_t k = b.active[ab];
-    const int ox0 = (k / (b.nby * b.nbz)) * kBinEdge, oy0 = ((k / b.nbz) % b.nby) * kBinEdge,
-              oz0 = (k % b.nbz) * kBinEdge;
-    for (int i = threadIdx.x; i < kP2gWaves * kTileNodes; i += kP2gThreads) wave_tiles[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int ox0 = (k / (b.nby * b.nbz)) * kCoarseEdge, oy0 = ((k / b.nbz) % b.nby) * kCoarseEdge,
+              oz0 = (k % b.nbz) * kCoarseEdge;
+    for (int i = threadIdx.x; i < kP2gWaves * Tile<kCoarseEdge>::kNodes; i += kP2gThreads) wave_tiles[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     const int32_t beg = b.offset[k], cnt = b.count[k];
     for (int32_t c0 = 0; c0 < cnt; c0 += kP2gChunk) {
       const int32_t n = min(kP2gChunk, cnt - c0);
@@ -937,7 +1030,7 @@ __global__ void __launch_bounds__(kP2gThreads, 2) k_mpm_p2g_cells(MpmArgs a, Bin
           for (int r = 0; r < 4; ++r) cur[r] = nxt[r];
         }
         if (np > 0u) {
-          const int lx = cl / (kBinEdge * kBinEdge), ly = (cl / kBinEdge) % kBinEdge, lz = cl % kBinEdge;
+          const int lx = cl / (kCoarseEdge * kCoarseEdge), ly = (cl / kCoarseEdge) % kCoarseEdge, lz = cl % kCoarseEdge;
 #pragma unroll
           for (int ox = 0; ox < 3; ++ox)
 #pragma unroll
@@ -946,51 +1039,134 @@ __global__ void __launch_bounds__(kP2gThreads, 2) k_mpm_p2g_cells(MpmArgs a, Bin
               for (int oz = 0; oz < 3; ++oz) {
                 const float* t = acc[(ox * 3 + oy) * 3 + oz];
                 const float md[3] = {t[1], t[2], t[3]};
-                tile_add(tile, ((lx + ox) * kTileEdge + (ly + oy)) * kTileEdge + (lz + oz), t[0], md);
+                tile_add(tile, ((lx + ox) * Tile<kCoarseEdge>::kEdge + (ly + oy)) * Tile<kCoarseEdge>::kEdge + (lz + oz), t[0], md);
               }
         }
       }
       __syncthreads();  // the cell tables and order are rewritten by the next chunk
     }
-    if (b.tiles) {
-      float* T = b.tiles + (size_t)k * kTileStride;
-      for (int i = threadIdx.x; i < kTileNodes; i += kP2gThreads) {
-        float4 v = wave_tiles[i];
+    flush_tiles<kCoarseEdge, kP2gWaves>(a, b, ab, ox0, oy0, oz0, wave_tiles);
+    __syncthreads();  // the wave tiles are cleared for the next block
+  }
+}
+
+// The same scatter of one block of 4^3 nodes: lane c of a wavefront takes cell c, over all chunks, so
+// the cells need no ordering by count and a cell's sums reach the tile once.  The bound is the chain
+// of dependent steps of a cell's particles, hence three wavefronts on a block, one per plane ox of
+// the stencil: the chain is a third as long, and 36 sums per lane instead of 108 let four wavefronts
+// share a SIMD.  The second and third wavefront's operand loads hit the cache.  (Staging a chunk's
+// operands in LDS in cell order instead was 1 us faster for 32^3 particles and 11 us slower for 100^3.)
+// 32^3 particles, 4.6 per cell: 66 us with 8^3 blocks, 12.3 us.
+constexpr int kFineWaves = 3;
+constexpr int kFineThreads = 64 * kFineWaves;
+constexpr int kFinePerThread = 5;
+constexpr int kFineChunk = kFinePerThread * kFineThreads;  // particles of a block ordered per pass
+static_assert(Tile<kFineEdge>::kCells == 64, "a block's cells are the lanes of a wavefront");
+static_assert(kFineChunk < 65536, "a particle's place in its cell is kept in 16 bits");
+
+// The contributions of a particle to plane ox of its stencil (p2g_scatter's arithmetic).
+template <typename Sink>
+__device__ inline void p2g_scatter_plane(const MpmArgs& a, const P2gPart& q, int ox, Sink sink) {
+  const float w0 = ox == 0 ? q.w[0][0] : ox == 1 ? q.w[0][1] : q.w[0][2];
+  const float dp0 = ((float)ox - q.fx[0]) * a.dx[0];
 #pragma unroll
-        for (int w = 1; w < kP2gWaves; ++w) {
-          const float4 u = wave_tiles[(size_t)w * kTileNodes + i];
-          v.x += u.x;
-          v.y += u.y;
-          v.z += u.z;
-          v.w += u.w;
-        }
-        T[i] = v.x;
-        T[kTileNodes + i] = v.y;
-        T[2 * kTileNodes + i] = v.z;
-        T[3 * kTileNodes + i] = v.w;
-      }
-    } else {
-      const uint32_t sx = (uint32_t)a.ny * a.nz, sy = a.nz;
-      for (int i = threadIdx.x; i < kTileNodes; i += kP2gThreads) {
-        const int tz = i % kTileEdge, ty = (i / kTileEdge) % kTileEdge, tx = i / (kTileEdge * kTileEdge);
-        const int gx = ox0 + tx, gy = oy0 + ty, gz = oz0 + tz;
-        if (gx >= a.nx || gy >= a.ny || gz >= a.nz) continue;
-        float4 v = wave_tiles[i];
+  for (int oy = 0; oy < 3; ++oy)
 #pragma unroll
-        for (int w = 1; w < kP2gWaves; ++w) {
-          const float4 u = wave_tiles[(size_t)w * kTileNodes + i];
-          v.x += u.x;
-          v.y += u.y;
-          v.z += u.z;
-          v.w += u.w;
-        }
-        const uint32_t node = (uint32_t)gx * sx + (uint32_t)gy * sy + (uint32_t)gz;
-        if (v.x != 0.0f) atomicAdd(&a.gm[node], v.x);
-        if (v.y != 0.0f) atomicAdd(&a.gv[3 * (size_t)node + 0], v.y);
-        if (v.z != 0.0f) atomicAdd(&a.gv[3 * (size_t)node + 1], v.z);
-        if (v.w != 0.0f) atomicAdd(&a.gv[3 * (size_t)node + 2], v.w);
-      }
+    for (int oz = 0; oz < 3; ++oz) {
+      const float wt = w0 * q.w[1][oy] * q.w[2][oz];
+      const float dp1 = ((float)oy - q.fx[1]) * a.dx[1];
+      const float dp2 = ((float)oz - q.fx[2]) * a.dx[2];
+      float md[3];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) md[d] = wt * (q.mom[d] + (q.aff[d][0] * dp0 + q.aff[d][1] * dp1 + q.aff[d][2] * dp2));
+      sink(oy, oz, wt * q.m, md);
     }
+}
+
+__global__ void __launch_bounds__(kFineThreads, 4) k_mpm_p2g_fine(MpmArgs a, BinArgs b) {
+  __shared__ float4 wave_tiles[kFineWaves * Tile<kFineEdge>::kNodes];  // mass, momentum
+  __shared__ uint32_t cell_count[Tile<kFineEdge>::kCells];
+  __shared__ uint32_t cell_start[Tile<kFineEdge>::kCells];  // first entry of each cell in order
+  __shared__ int32_t order[kFineChunk];          // the chunk's particles by cell
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63u);
+  float4* tile = wave_tiles + wave * Tile<kFineEdge>::kNodes;
+  const ChunkRange cr = xcd_chunks((uint32_t)*b.nactive);
+  for (uint32_t ab = cr.first; ab < cr.end; ab += cr.step) {
+    const int32_t k = b.active[ab];
+    const int ox0 = (k / (b.nby * b.nbz)) * kFineEdge, oy0 = ((k / b.nbz) % b.nby) * kFineEdge,
+              oz0 = (k % b.nbz) * kFineEdge;
+    for (int i = threadIdx.x; i < kFineWaves * Tile<kFineEdge>::kNodes; i += kFineThreads) wave_tiles[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int32_t beg = b.offset[k], cnt = b.count[k];
+    float acc[9][4];
+#pragma unroll
+    for (int o = 0; o < 9; ++o) acc[o][0] = acc[o][1] = acc[o][2] = acc[o][3] = 0.0f;
+    for (int32_t c0 = 0; c0 < cnt; c0 += kFineChunk) {
+      const int32_t n = min(kFineChunk, cnt - c0);
+      if (threadIdx.x < Tile<kFineEdge>::kCells) cell_count[threadIdx.x] = 0u;
+      __syncthreads();
+      uint32_t place[kFinePerThread];
+      int32_t part[kFinePerThread];
+#pragma unroll
+      for (int j = 0; j < kFinePerThread; ++j) {
+        const int t = (int)threadIdx.x + j * kFineThreads;
+        place[j] = t < n ? (uint32_t)b.scell[beg + c0 + t] : 0u;
+        part[j] = t < n ? b.sorted[beg + c0 + t] : 0;
+      }
+#pragma unroll
+      for (int j = 0; j < kFinePerThread; ++j) {
+        const int t = (int)threadIdx.x + j * kFineThreads;
+        if (t < n) place[j] = (place[j] << 16) | atomicAdd(&cell_count[place[j]], 1u);
+      }
+      __syncthreads();
+      // every wavefront scans the 64 counts: lane c keeps the range of cell c
+      const uint32_t np = cell_count[lane];
+      uint32_t incl = np;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += y;
+      }
+      const uint32_t s = incl - np;
+      if (wave == 0) cell_start[lane] = s;
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kFinePerThread; ++j) {
+        const int t = (int)threadIdx.x + j * kFineThreads;
+        if (t < n) order[cell_start[place[j] >> 16] + (place[j] & 0xffffu)] = part[j];
+      }
+      __syncthreads();
+      float4 cur[4] = {};
+      if (np > 0u) load_stage(b.stage, order[s], cur);
+      for (uint32_t i = 0; i < np; ++i) {
+        float4 nxt[4] = {};
+        if (i + 1u < np) load_stage(b.stage, order[s + i + 1u], nxt);
+        P2gPart q;
+        p2g_unstage(cur, q);
+        p2g_scatter_plane(a, q, wave, [&](int oy, int oz, float mw, const float (&md)[3]) {
+          float* t = acc[oy * 3 + oz];
+          t[0] += mw;
+          t[1] += md[0];
+          t[2] += md[1];
+          t[3] += md[2];
+        });
+#pragma unroll
+        for (int r = 0; r < 4; ++r) cur[r] = nxt[r];
+      }
+      __syncthreads();  // the cell tables and order are rewritten by the next chunk
+    }
+    {
+      const int lx = lane / (kFineEdge * kFineEdge), ly = (lane / kFineEdge) % kFineEdge, lz = lane % kFineEdge;
+#pragma unroll
+      for (int oy = 0; oy < 3; ++oy)
+#pragma unroll
+        for (int oz = 0; oz < 3; ++oz) {
+          const float* t = acc[oy * 3 + oz];
+          const float md[3] = {t[1], t[2], t[3]};
+          tile_add(tile, ((lx + wave) * Tile<kFineEdge>::kEdge + (ly + oy)) * Tile<kFineEdge>::kEdge + (lz + oz), t[0], md);
+        }
+    }
+    __syncthreads();
+    flush_tiles<kFineEdge, kFineWaves>(a, b, ab, ox0, oy0, oz0, wave_tiles);
     __syncthreads();  // the wave tiles are cleared for the next block
   }
 }
@@ -998,17 +1174,19 @@ __global__ void __launch_bounds__(kP2gThreads, 2) k_mpm_p2g_cells(MpmArgs a, Bin
 // External-force part of the binned P2G: f += w f_ext over the 27 nodes of every particle with a
 // non-zero force (fixed particles carry none), LDS atomics into a block tile.  A block without
 // such particles writes no force components and is flagged so that the grid update skips them.
+template <int EDGE>
 __global__ void __launch_bounds__(kBlock) k_mpm_p2g_force(MpmArgs a, BinArgs b) {
-  __shared__ float tf[3][kTileNodes];
+  constexpr int kNodes = Tile<EDGE>::kNodes, kEdge = Tile<EDGE>::kEdge;
+  __shared__ float tf[3][kNodes];
   __shared__ int32_t any;
-  const int32_t nact = *b.nactive;
   const uint32_t sx = (uint32_t)a.ny * a.nz, sy = a.nz;
-  for (int32_t ab = blockIdx.x; ab < nact; ab += gridDim.x) {
+  const ChunkRange cr = xcd_chunks((uint32_t)*b.nactive);
+  for (uint32_t ab = cr.first; ab < cr.end; ab += cr.step) {
     const int32_t k = b.active[ab];
-    const int ox0 = (k / (b.nby * b.nbz)) * kBinEdge, oy0 = ((k / b.nbz) % b.nby) * kBinEdge,
-              oz0 = (k % b.nbz) * kBinEdge;
+    const int ox0 = (k / (b.nby * b.nbz)) * EDGE, oy0 = ((k / b.nbz) % b.nby) * EDGE,
+              oz0 = (k % b.nbz) * EDGE;
     if (threadIdx.x == 0) any = 0;
-    for (int i = threadIdx.x; i < kTileNodes; i += kBlock) tf[0][i] = tf[1][i] = tf[2][i] = 0.0f;
+    for (int i = threadIdx.x; i < kNodes; i += kBlock) tf[0][i] = tf[1][i] = tf[2][i] = 0.0f;
     __syncthreads();
     const int32_t beg = b.offset[k], cnt = b.count[k];
     for (int32_t t = threadIdx.x; t < cnt; t += kBlock) {
@@ -1033,7 +1211,7 @@ __global__ void __launch_bounds__(kBlock) k_mpm_p2g_force(MpmArgs a, BinArgs b) 
 #pragma unroll
           for (int oz = 0; oz < 3; ++oz) {
             const float wt = w[0][ox] * w[1][oy] * w[2][oz];
-            const int li = ((lx + ox) * kTileEdge + (ly + oy)) * kTileEdge + (lz + oz);
+            const int li = ((lx + ox) * kEdge + (ly + oy)) * kEdge + (lz + oz);
 #pragma unroll
             for (int d = 0; d < 3; ++d)
               if (fe[d] != 0.0f) atomicAdd(&tf[d][li], wt * fe[d]);
@@ -1042,14 +1220,14 @@ __global__ void __launch_bounds__(kBlock) k_mpm_p2g_force(MpmArgs a, BinArgs b) 
     __syncthreads();
     if (any) {
       if (b.tiles) {
-        float* T = b.tiles + (size_t)k * kTileStride;
-        for (int i = threadIdx.x; i < kTileNodes; i += kBlock) {
+        float* T = b.tiles + (size_t)ab * Tile<EDGE>::kStride;
+        for (int i = threadIdx.x; i < kNodes; i += kBlock) {
 #pragma unroll
-          for (int d = 0; d < 3; ++d) T[(4 + d) * kTileNodes + i] = tf[d][i];
+          for (int d = 0; d < 3; ++d) T[(4 + d) * kNodes + i] = tf[d][i];
         }
       } else {
-        for (int i = threadIdx.x; i < kTileNodes; i += kBlock) {
-          const int tz = i % kTileEdge, ty = (i / kTileEdge) % kTileEdge, tx = i / (kTileEdge * kTileEdge);
+        for (int i = threadIdx.x; i < kNodes; i += kBlock) {
+          const int tz = i % kEdge, ty = (i / kEdge) % kEdge, tx = i / (kEdge * kEdge);
           const int gx = ox0 + tx, gy = oy0 + ty, gz = oz0 + tz;
           if (gx >= a.nx || gy >= a.ny || gz >= a.nz) continue;
           const uint32_t node = (uint32_t)gx * sx + (uint32_t)gy * sy + (uint32_t)gz;
@@ -1059,32 +1237,31 @@ __global__ void __launch_bounds__(kBlock) k_mpm_p2g_force(MpmArgs a, BinArgs b) 
         }
       }
     }
-    if (threadIdx.x == 0 && b.block_force) b.block_force[k] = any;
+    if (threadIdx.x == 0 && b.block_force) b.block_force[ab] = any;
     __syncthreads();  // the tile and the flag are reused by the next block
   }
 }
 
 // Blocks of the previous step's need list that this step does not list: zero their nodes (every
 // node outside the need list is zero, and the grid update rewrites every node of the listed blocks).
-__global__ void __launch_bounds__(kBlock) k_clear_stale(MpmArgs a, BinArgs b) {
-  const int32_t n = *b.nprev;
-  const uint32_t sx = (uint32_t)a.ny * a.nz, sy = a.nz;
-  constexpr int kBlockNodes = kBinEdge * kBinEdge * kBinEdge;
-  for (int32_t w = blockIdx.x; w < n; w += gridDim.x) {
-    const int32_t B = b.prev_need[w];
+// A wavefront takes 64 nodes of a block: units first, first + step, ... of the list.
+template <int EDGE>
+__device__ inline void clear_stale(const MpmArgs& a, const BinArgs& b, uint32_t first, uint32_t step) {
+  constexpr uint32_t kUnits = Tile<EDGE>::kCells / 64;
+  const uint32_t n = (uint32_t)*b.nprev * kUnits;
+  for (uint32_t w = first; w < n; w += step) {
+    const int32_t B = b.prev_need[w / kUnits];
     if (b.need_stamp[B] == b.stamp) continue;
-    const int32_t bx = B / (b.nby * b.nbz), by = (B / b.nbz) % b.nby, bz = B % b.nbz;
-    for (int t = threadIdx.x; t < kBlockNodes; t += blockDim.x) {
-      const int gx = bx * kBinEdge + t / (kBinEdge * kBinEdge), gy = by * kBinEdge + (t / kBinEdge) % kBinEdge,
-                gz = bz * kBinEdge + t % kBinEdge;
-      if (gx >= a.nx || gy >= a.ny || gz >= a.nz) continue;
-      const uint32_t node = (uint32_t)gx * sx + (uint32_t)gy * sy + (uint32_t)gz;
-      a.gm[node] = 0.0f;
+    const int t = (int)(w % kUnits * 64 + (threadIdx.x & 63u));
+    const int gx = (B / (b.nby * b.nbz)) * EDGE + t / (EDGE * EDGE), gy = ((B / b.nbz) % b.nby) * EDGE + (t / EDGE) % EDGE,
+              gz = (B % b.nbz) * EDGE + t % EDGE;
+    if (gx >= a.nx || gy >= a.ny || gz >= a.nz) continue;
+    const size_t node = ((size_t)gx * a.ny + gy) * a.nz + gz;
+    a.gm[node] = 0.0f;
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        a.gv[3 * (size_t)node + d] = 0.0f;
-        a.gf[3 * (size_t)node + d] = 0.0f;
-      }
+    for (int d = 0; d < 3; ++d) {
+      a.gv[3 * node + d] = 0.0f;
+      a.gf[3 * node + d] = 0.0f;
     }
   }
 }
@@ -1120,61 +1297,98 @@ __global__ void __launch_bounds__(kBlock) k_mpm_grid(MpmArgs a) {
 // that cover it (its own block's and, within 2 nodes of a low face, the lower
 // neighbours'), in a fixed order, then updates as k_mpm_grid and writes mass,
 // velocity and force.  Nodes of listed blocks without mass get the raw sums
-// (zero), as the cleared grid has.  Totals 12..19.
+// (zero), as the cleared grid has.  Totals 12..19.  One wavefront per 64 nodes of a block; the
+// (up to) eight tiles' values are loaded together and added afterwards, so that a node costs one
+// memory round trip after the list's, not eight.  The last kStaleGroups workgroups clear the nodes
+// of the blocks that only the previous step listed.
+constexpr uint32_t kStaleGroups = 64;
+
+template <int EDGE>
 __global__ void __launch_bounds__(kBlock) k_mpm_grid_gather(MpmArgs a, BinArgs b) {
   constexpr int NS = 8;
+  constexpr int kWaves = kBlock / 64, kNodes = Tile<EDGE>::kNodes, kEdge = Tile<EDGE>::kEdge;
+  constexpr uint32_t kUnits = Tile<EDGE>::kCells / 64;
   __shared__ double lds[NS * (kBlock / 64)];
+  const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63u);
+  const uint32_t groups = gridDim.x - kStaleGroups;
+  if (blockIdx.x >= groups) {
+    clear_stale<EDGE>(a, b, (blockIdx.x - groups) * kWaves + (uint32_t)wave, kStaleGroups * kWaves);
+    return;
+  }
   double acc[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) acc[s] = 0.0;
-  const int32_t nneed = *b.nneed;
-  const uint32_t sx = (uint32_t)a.ny * a.nz, sy = a.nz;
-  constexpr int kBlockNodes = kBinEdge * kBinEdge * kBinEdge;
-  for (int32_t w = blockIdx.x; w < nneed; w += gridDim.x) {
-    const int32_t B = b.need_list[w];
+  const uint32_t nneed = (uint32_t)*b.nneed * kUnits;
+  const ChunkRange cr = xcd_chunks((nneed + kWaves - 1) / kWaves, groups);
+  for (uint32_t ch = cr.first; ch < cr.end; ch += cr.step) {
+    const uint32_t w = ch * kWaves + (uint32_t)wave;
+    if (w >= nneed) break;
+    const int32_t B = b.need_list[w / kUnits];
+    const int t = (int)(w % kUnits) * 64 + lane;
+    const int lx = t / (EDGE * EDGE), ly = (t / EDGE) % EDGE, lz = t % EDGE;
     const int32_t bx = B / (b.nby * b.nbz), by = (B / b.nbz) % b.nby, bz = B % b.nbz;
-    for (int t = threadIdx.x; t < kBlockNodes; t += blockDim.x) {
-      const int lx = t / (kBinEdge * kBinEdge), ly = (t / kBinEdge) % kBinEdge, lz = t % kBinEdge;
-      const int gx = bx * kBinEdge + lx, gy = by * kBinEdge + ly, gz = bz * kBinEdge + lz;
-      if (gx >= a.nx || gy >= a.ny || gz >= a.nz) continue;
-      float m = 0.0f, p[3] = {0.0f, 0.0f, 0.0f}, f[3] = {0.0f, 0.0f, 0.0f};
+    const int gx = bx * EDGE + lx, gy = by * EDGE + ly, gz = bz * EDGE + lz;
+    if (gx >= a.nx || gy >= a.ny || gz >= a.nz) continue;
+    int32_t slot[8];  // of the covering tile, or -1
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int ex = e >> 2, ey = (e >> 1) & 1, ez = e & 1;
+      const bool in = bx >= ex && by >= ey && bz >= ez;
+      const int32_t k = in ? B - (ex * b.nby + ey) * b.nbz - ez : B;
+      const bool covers = in && (!ex || lx < 2) && (!ey || ly < 2) && (!ez || lz < 2) && b.count[k] > 0;
+      slot[e] = covers ? b.slot[k] : -1;
+    }
+    float tv[8][4];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int ex = e >> 2, ey = (e >> 1) & 1, ez = e & 1;
+      const int ti = ((lx + ex * EDGE) * kEdge + (ly + ey * EDGE)) * kEdge + (lz + ez * EDGE);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) tv[e][c] = 0.0f;
+      if (slot[e] >= 0) {
+        const float* T = b.tiles + (size_t)slot[e] * Tile<EDGE>::kStride + ti;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) tv[e][c] = T[c * kNodes];
+      }
+    }
+    float f[3] = {0.0f, 0.0f, 0.0f};
+    if (b.has_force) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int ex = e >> 2, ey = (e >> 1) & 1, ez = e & 1;
-        if ((ex && lx >= 2) || (ey && ly >= 2) || (ez && lz >= 2)) continue;
-        if (bx - ex < 0 || by - ey < 0 || bz - ez < 0) continue;
-        const int32_t k = ((bx - ex) * b.nby + (by - ey)) * b.nbz + (bz - ez);
-        if (b.count[k] <= 0) continue;
-        const float* T = b.tiles + (size_t)k * kTileStride;
-        const int ti = ((lx + ex * kBinEdge) * kTileEdge + (ly + ey * kBinEdge)) * kTileEdge + (lz + ez * kBinEdge);
-        m += T[ti];
+        const int ti = ((lx + ex * EDGE) * kEdge + (ly + ey * EDGE)) * kEdge + (lz + ez * EDGE);
+        if (slot[e] < 0 || !b.block_force[slot[e]]) continue;
+        const float* T = b.tiles + (size_t)slot[e] * Tile<EDGE>::kStride + ti;
 #pragma unroll
-        for (int d = 0; d < 3; ++d) p[d] += T[(1 + d) * kTileNodes + ti];
-        if (b.has_force && b.block_force[k]) {
-#pragma unroll
-          for (int d = 0; d < 3; ++d) f[d] += T[(4 + d) * kTileNodes + ti];
-        }
+        for (int d = 0; d < 3; ++d) f[d] += T[(4 + d) * kNodes];
       }
-      const uint32_t node = (uint32_t)gx * sx + (uint32_t)gy * sy + (uint32_t)gz;
-      a.gm[node] = m;
-      float v[3] = {p[0], p[1], p[2]};
-      if (m > 1.0e-20f) {
+    }
+    float m = 0.0f, p[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          v[d] = p[d] / m;
-          v[d] += a.dt * f[d] / m;
-          acc[d] += (double)(m * v[d]);
-          v[d] *= a.damping;
-          acc[3 + d] += (double)(m * v[d]);
-        }
-        acc[6] += 1.0;
-        acc[7] = fmax(acc[7], (double)sqrtf(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]));
-      }
+    for (int e = 0; e < 8; ++e) {
+      m += tv[e][0];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) p[d] += tv[e][1 + d];
+    }
+    const size_t node = ((size_t)gx * a.ny + gy) * a.nz + gz;
+    a.gm[node] = m;
+    float v[3] = {p[0], p[1], p[2]};
+    if (m > 1.0e-20f) {
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        a.gv[3 * (size_t)node + d] = v[d];
-        a.gf[3 * (size_t)node + d] = f[d];
+        v[d] = p[d] / m;
+        v[d] += a.dt * f[d] / m;
+        acc[d] += (double)(m * v[d]);
+        v[d] *= a.damping;
+        acc[3 + d] += (double)(m * v[d]);
       }
+      acc[6] += 1.0;
+      acc[7] = fmax(acc[7], (double)sqrtf(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]));
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      a.gv[3 * node + d] = v[d];
+      a.gf[3 * node + d] = f[d];
     }
   }
   mpm_partials<NS>(acc, a, a.prow0 + blockIdx.x, lds, kGridMax);
@@ -1204,6 +1418,23 @@ __device__ inline void update_surface(const MpmArgs& a, uint32_t p) {
 }
 
 __device__ inline void g2p_report(const MpmArgs& a, uint32_t p, double (&acc)[21]);
+
+// The part of a particle's G2P that needs no grid: the reset of a fixed particle and the surface.
+__device__ inline void g2p_rest(const MpmArgs& a, uint32_t p, bool fixed) {
+  if (fixed) {
+    float* vp = a.v + 3 * (size_t)p;
+    float* Cp = a.C + 9 * (size_t)p;
+    float* Fp = a.F + 9 * (size_t)p;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) vp[d] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+      Cp[i] = 0.0f;
+      Fp[i] = (i % 4 == 0) ? 1.0f : 0.0f;
+    }
+  }
+  update_surface(a, p);
+}
 
 // G2P of one particle (neo_hookean_mpm.py:819-874) with the grid velocity of node base + (ox, oy, oz)
 // from vel(base, ox, oy, oz, out[3]); with SUMS, its report totals 20..40 into acc (g2p_report).
@@ -1271,19 +1502,7 @@ __device__ inline void g2p_particle(const MpmArgs& a, uint32_t p, double (&acc)[
         }
     }
   }
-  if (fixed) {
-    float* vp = a.v + 3 * (size_t)p;
-    float* Cp = a.C + 9 * (size_t)p;
-    float* Fp = a.F + 9 * (size_t)p;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) vp[d] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-      Cp[i] = 0.0f;
-      Fp[i] = (i % 4 == 0) ? 1.0f : 0.0f;
-    }
-  }
-  update_surface(a, p);
+  g2p_rest(a, p, fixed);
   if (SUMS) g2p_report(a, p, acc);
 }
 
@@ -1345,19 +1564,34 @@ __global__ void __launch_bounds__(kBlock) k_mpm_g2p(MpmArgs a) {
   mpm_partials<NS>(acc, a, a.prow0 + blockIdx.x, lds, 0ull);
 }
 
-// G2P of the binned path: per active block, the 10^3 grid velocities its particles' stencils reach
-// are staged in LDS and the block's particles gather from there.  Totals 20..40.
+// G2P of the binned path: per active block, the grid velocities its particles' stencils reach
+// are staged in LDS and the block's particles gather from there.  The last kOobGroups workgroups take
+// the out-of-bounds particles (no gather: fixed-particle reset and surface update; they stay outside
+// the grid, so they add nothing to the report sums).  The report sums are k_mpm_g2p_sums'.
+constexpr uint32_t kOobGroups = 16;
+
+template <int EDGE>
 __global__ void __launch_bounds__(kBlock, 4) k_mpm_g2p_binned(MpmArgs a, BinArgs b) {
-  __shared__ float tv[3][kTileNodes];
+  constexpr int kNodes = Tile<EDGE>::kNodes, kEdge = Tile<EDGE>::kEdge;
+  __shared__ float tv[3][kNodes];
   double none[21];  // report sums: k_mpm_g2p_sums
-  const int32_t nact = *b.nactive;
   const uint32_t sx = (uint32_t)a.ny * a.nz, sy = a.nz;
-  for (int32_t ab = blockIdx.x; ab < nact; ab += gridDim.x) {
+  const uint32_t groups = gridDim.x - kOobGroups;
+  if (blockIdx.x >= groups) {
+    const int32_t n = *b.noob;
+    for (int32_t i = (int32_t)((blockIdx.x - groups) * kBlock + threadIdx.x); i < n; i += (int32_t)kOobGroups * kBlock) {
+      const uint32_t p = (uint32_t)b.oob[i];
+      g2p_rest(a, p, a.fixed && a.fixed[p] != 0);
+    }
+    return;
+  }
+  const ChunkRange cr = xcd_chunks((uint32_t)*b.nactive, groups);
+  for (uint32_t ab = cr.first; ab < cr.end; ab += cr.step) {
     const int32_t k = b.active[ab];
-    const int ox0 = (k / (b.nby * b.nbz)) * kBinEdge, oy0 = ((k / b.nbz) % b.nby) * kBinEdge,
-              oz0 = (k % b.nbz) * kBinEdge;
-    for (int i = threadIdx.x; i < kTileNodes; i += kBlock) {
-      const int tz = i % kTileEdge, ty = (i / kTileEdge) % kTileEdge, tx = i / (kTileEdge * kTileEdge);
+    const int ox0 = (k / (b.nby * b.nbz)) * EDGE, oy0 = ((k / b.nbz) % b.nby) * EDGE,
+              oz0 = (k % b.nbz) * EDGE;
+    for (int i = threadIdx.x; i < kNodes; i += kBlock) {
+      const int tz = i % kEdge, ty = (i / kEdge) % kEdge, tx = i / (kEdge * kEdge);
       const int gx = ox0 + tx, gy = oy0 + ty, gz = oz0 + tz;
       const bool inside = gx < a.nx && gy < a.ny && gz < a.nz;
       const size_t node = inside ? (size_t)gx * sx + (size_t)gy * sy + (size_t)gz : 0;
@@ -1366,7 +1600,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_mpm_g2p_binned(MpmArgs a, BinArgs
     }
     __syncthreads();
     auto vel = [&](const int (&base)[3], int ox, int oy, int oz, float (&out)[3]) {
-      const int li = ((base[0] - ox0 + ox) * kTileEdge + (base[1] - oy0 + oy)) * kTileEdge + (base[2] - oz0 + oz);
+      const int li = ((base[0] - ox0 + ox) * kEdge + (base[1] - oy0 + oy)) * kEdge + (base[2] - oz0 + oz);
 #pragma unroll
       for (int d = 0; d < 3; ++d) out[d] = tv[d][li];
     };
@@ -1374,21 +1608,6 @@ __global__ void __launch_bounds__(kBlock, 4) k_mpm_g2p_binned(MpmArgs a, BinArgs
     for (int32_t t = threadIdx.x; t < cnt; t += kBlock) g2p_particle<false>(a, (uint32_t)b.sorted[beg + t], none, vel);
     __syncthreads();  // the velocity tile is reloaded for the next block
   }
-}
-
-// G2P of the binned path's out-of-bounds particles (no gather: fixed-particle reset and surface
-// update; they stay outside the grid, so they add nothing to the report sums).
-__global__ void __launch_bounds__(kBlock) k_mpm_g2p_oob(MpmArgs a, BinArgs b) {
-  double none[21];
-  const int32_t n = *b.noob;
-  const uint32_t sx = (uint32_t)a.ny * a.nz, sy = a.nz;
-  auto vel = [&](const int (&base)[3], int ox, int oy, int oz, float (&out)[3]) {
-    const uint32_t node = (uint32_t)(base[0] + ox) * sx + (uint32_t)(base[1] + oy) * sy + (uint32_t)(base[2] + oz);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) out[d] = a.gv[3 * (size_t)node + d];
-  };
-  for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    g2p_particle<false>(a, (uint32_t)b.oob[i], none, vel);
 }
 
 // Report totals 20..40 of the binned G2P, over every particle in particle order after the update.
@@ -1437,10 +1656,6 @@ __global__ void __launch_bounds__(kBlock) k_mpm_radial(MpmArgs a) {
 
 }
 
-
-struct FinNone {
-  __device__ void operator()(const double*) const {}
-};
 
 // Report snapshot (neo_hookean_mpm.py:899-959) from the stage totals, run by
 // the finishing workgroup of the radial-stretch reduction.
@@ -1737,16 +1952,22 @@ int hfsi_mpm_create(hfsi_mpm** out, int32_t capacity, const double* bounds_min3,
   }
   {
     BinArgs& b = h->bins;
-    b.nbx = (h->nx + kBinEdge - 1) / kBinEdge;
-    b.nby = (h->ny + kBinEdge - 1) / kBinEdge;
-    b.nbz = (h->nz + kBinEdge - 1) / kBinEdge;
-    const size_t nb = (size_t)b.nbx * b.nby * b.nbz;
-    const size_t nchunks = (nb + kScanChunk - 1) / kScanChunk;
-    if (nchunks > (size_t)kScanChunk) {
+    auto blocks = [&](int edge) {
+      b.edge = edge;
+      b.nbx = (h->nx + edge - 1) / edge;
+      b.nby = (h->ny + edge - 1) / edge;
+      b.nbz = (h->nz + edge - 1) / edge;
+      return (size_t)b.nbx * b.nby * b.nbz;
+    };
+    size_t nb = blocks(kCoarseEdge);
+    if (nb > kMaxBlocks) {
       set_error("hfsi_mpm_create: grid too large for the particle binning");
       hfsi_mpm_destroy(h);
       return HFSI_ERR_ARG;
     }
+    const bool with_tiles = nb <= kMaxTileBlocks;
+    const bool fine = capacity <= kFineParticles;
+    if (fine) nb = blocks(kFineEdge);
     auto al = [&](int32_t** p, size_t n) {
       void* q = nullptr;
       if (hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(int32_t)) != hipSuccess) return false;
@@ -1758,18 +1979,20 @@ int hfsi_mpm_create(hfsi_mpm** out, int32_t capacity, const double* bounds_min3,
     int32_t* stage = nullptr;
     if (!(al(&b.key, P) && al(&b.rank, P) && al(&b.count, nb) && al(&b.offset, nb) && al(&b.sorted, P) &&
           al(&b.active, nb) && al(&b.nactive, 1) && al(&b.oob, P) && al(&b.noob, 1) && al(&b.svd, P) &&
-          al(&b.nsvd, 1) && al(&b.scan_sums, nchunks) &&
+          al(&b.nsvd, 1) && al(&b.slot, nb) && al(&b.nsorted, 1) &&
           al(&b.cell, P) && al(&b.scell, P) && al(&stage, 16 * P))) {
       set_error("hfsi_mpm_create: device allocation failed");
       hfsi_mpm_destroy(h);
       return HFSI_ERR_HIP;
     }
     b.stage = (float4*)stage;  // hipMalloc memory: 256-byte aligned
-    if (nb <= kMaxTileBlocks) {
+    if (with_tiles) {
+      const size_t stride = fine ? Tile<kFineEdge>::kStride : Tile<kCoarseEdge>::kStride;
+      const size_t tiles = std::min(nb, P);  // blocks that can be active together
       void* q = nullptr;
       if (!(al(&b.need_stamp, nb) && al(&b.need_list, nb) && al(&b.nneed, 1) && al(&b.prev_need, nb) &&
-            al(&b.nprev, 1) && al(&b.block_force, nb) && hipMemset(b.nprev, 0, sizeof(int32_t)) == hipSuccess &&
-            hipMalloc(&q, nb * kTileStride * sizeof(float)) == hipSuccess &&
+            al(&b.nprev, 1) && al(&b.block_force, tiles) && hipMemset(b.nprev, 0, sizeof(int32_t)) == hipSuccess &&
+            hipMalloc(&q, tiles * stride * sizeof(float)) == hipSuccess &&
             hipMemset(b.need_stamp, 0, nb * sizeof(int32_t)) == hipSuccess)) {
         set_error("hfsi_mpm_create: device allocation failed");
         if (q) (void)hipFree(q);
@@ -1865,6 +2088,7 @@ int hfsi_mpm_step(hfsi_mpm* h, const hfsi_mpm_particles* P, int32_t count, const
   BinArgs& b = h->bins;
   const bool binned = h->p2g_mode == HFSI_MPM_P2G_BINNED;
   const bool tile_path = binned && b.tiles != nullptr;
+  const bool fine = b.edge == kFineEdge;
   const bool same_grid = h->tracked_grid[0] == G->mass && h->tracked_grid[1] == G->velocity &&
                          h->tracked_grid[2] == G->force;
   // The tile path rewrites every node of the blocks it lists and zeroes the blocks it listed last
@@ -1872,73 +2096,75 @@ int hfsi_mpm_step(hfsi_mpm* h, const hfsi_mpm_particles* P, int32_t count, const
   const bool full_clear = !tile_path || !h->grid_tracked || !same_grid;
   if (full_clear)
     hipLaunchKernelGGL(k_mpm_clear, dim3(mpm_blocks(nodes)), dim3(kBlock), 0, st, nodes, a.gm, a.gv, a.gf);
-  // each reduction stage: its kernels' workgroups write rows [prow0, prow0 + grid) of one slot-major
-  // table of `pstride` rows, which one workgroup then combines
+  // each reduction stage: its kernels' workgroups write rows [prow0, prow0 + grid) of a slot-major
+  // table of `pstride` rows of its own, which one workgroup then combines
+  double* table = h->partials;
   auto rows = [&](uint32_t row0, uint32_t stride) {
+    a.partials = table;
     a.prow0 = row0;
     a.pstride = stride;
   };
-  const uint32_t GP = binned ? (uint32_t)std::min<int32_t>(b.nbx * b.nby * b.nbz, 1024) : 0u, GO = 64;
+  auto next_table = [&](uint32_t nrows, uint32_t slots) {
+    const StageRows t{table, nrows};
+    table += (size_t)nrows * slots;
+    return t;
+  };
+  // workgroups of the per-block kernels: one per block that can be active, up to 4096 (16 per CU)
+  const int64_t can_be_active = std::min<int64_t>((int64_t)b.nbx * b.nby * b.nbz, count);
+  const uint32_t GP = (uint32_t)(std::min<int64_t>(can_be_active, 4096) + HFSI_NXCD - 1) / HFSI_NXCD * HFSI_NXCD;
+  const uint32_t GO = 64;
+  StageRows p2g_rows{}, grid_rows{}, g2p_rows{};
   if (binned) {
     b.stamp = b.stamp == INT32_MAX ? 1 : b.stamp + 1;
     b.has_force = a.f_ext != nullptr;
     const int32_t nblk = b.nbx * b.nby * b.nbz;
-    const int32_t nchunks = (nblk + kScanChunk - 1) / kScanChunk;
     b.reset_prev = full_clear ? 1 : 0;
     hipLaunchKernelGGL(k_bin_clear, dim3(std::min<int32_t>((nblk + 255) / 256, 1024)), dim3(256), 0, st, b);
-    hipLaunchKernelGGL(k_bin_count, dim3(pbin), dim3(kBlock), 0, st, a, b);
-    hipLaunchKernelGGL(k_scan_chunks, dim3(nchunks), dim3(kScanChunk), 0, st, (const int32_t*)b.count, b.offset,
-                       nblk, b.scan_sums);
-    hipLaunchKernelGGL(k_scan_add, dim3(nchunks), dim3(kScanChunk), 0, st, b.offset, nblk,
-                       (const int32_t*)b.scan_sums, nchunks);
+    hipLaunchKernelGGL(fine ? k_bin_count<kFineEdge> : k_bin_count<kCoarseEdge>, dim3(pbin), dim3(kBlock), 0, st, a, b);
+    hipLaunchKernelGGL(k_bin_lists, dim3((nblk + kListBlocks - 1) / kListBlocks), dim3(kListBlocks), 0, st, b);
     hipLaunchKernelGGL(k_bin_scatter, dim3(pbin), dim3(kBlock), 0, st, count, b);
-    if (tile_path) {
-      hipLaunchKernelGGL(k_need_mark, dim3(std::min<int32_t>((nblk + 255) / 256, 256)), dim3(256), 0, st, b);
-      hipLaunchKernelGGL(k_clear_stale, dim3(1024), dim3(kBlock), 0, st, a, b);
-    }
     rows(0, pb + GO);
     hipLaunchKernelGGL(k_mpm_p2g_prepare, dim3(pb), dim3(kBlock), 0, st, a, b);
     rows(pb, pb + GO);
     hipLaunchKernelGGL(k_mpm_p2g_prepare_svd, dim3(GO), dim3(kBlock), 0, st, a, b);
-    hipLaunchKernelGGL((k_mpm_finish<12, FinNone>), dim3(1), dim3(kMpmFinishThreads), 0, st, (const double*)a.partials,
-                       pb + GO, pb + GO, a.totals + 0, FinNone{}, kP2gMax);
-    hipLaunchKernelGGL(k_mpm_p2g_cells, dim3(GP), dim3(kP2gThreads), kP2gTileBytes, st, a, b);
-    if (b.has_force) hipLaunchKernelGGL(k_mpm_p2g_force, dim3(GP), dim3(kBlock), 0, st, a, b);
+    p2g_rows = next_table(pb + GO, 12);
+    if (fine)
+      hipLaunchKernelGGL(k_mpm_p2g_fine, dim3(GP), dim3(kFineThreads), 0, st, a, b);
+    else
+      hipLaunchKernelGGL(k_mpm_p2g_cells, dim3(GP), dim3(kP2gThreads), kP2gTileBytes, st, a, b);
+    if (b.has_force)
+      hipLaunchKernelGGL(fine ? k_mpm_p2g_force<kFineEdge> : k_mpm_p2g_force<kCoarseEdge>, dim3(GP), dim3(kBlock), 0, st,
+                         a, b);
   } else {
     rows(0, pb);
     hipLaunchKernelGGL(k_mpm_p2g, dim3(pb), dim3(kBlock), 0, st, a);
-    hipLaunchKernelGGL((k_mpm_finish<12, FinNone>), dim3(1), dim3(kMpmFinishThreads), 0, st, (const double*)a.partials,
-                       pb, pb, a.totals + 0, FinNone{}, kP2gMax);
+    p2g_rows = next_table(pb, 12);
   }
   if (tile_path) {
     const uint32_t GG = 1024;
     rows(0, GG);
-    hipLaunchKernelGGL(k_mpm_grid_gather, dim3(GG), dim3(kBlock), 0, st, a, b);
-    hipLaunchKernelGGL((k_mpm_finish<8, FinNone>), dim3(1), dim3(kMpmFinishThreads), 0, st, (const double*)a.partials,
-                       GG, GG, a.totals + T_TRANS, FinNone{}, kGridMax);
+    hipLaunchKernelGGL(fine ? k_mpm_grid_gather<kFineEdge> : k_mpm_grid_gather<kCoarseEdge>, dim3(GG + kStaleGroups), dim3(kBlock), 0, st, a, b);
+    grid_rows = next_table(GG, 8);
   } else {
     rows(0, nb);
     hipLaunchKernelGGL(k_mpm_grid, dim3(nb), dim3(kBlock), 0, st, a);
-    hipLaunchKernelGGL((k_mpm_finish<8, FinNone>), dim3(1), dim3(kMpmFinishThreads), 0, st, (const double*)a.partials,
-                       nb, nb, a.totals + T_TRANS, FinNone{}, kGridMax);
+    grid_rows = next_table(nb, 8);
   }
-  if (binned) {
-    hipLaunchKernelGGL(k_mpm_g2p_binned, dim3(GP), dim3(kBlock), 0, st, a, b);
-    hipLaunchKernelGGL(k_mpm_g2p_oob, dim3(GO), dim3(kBlock), 0, st, a, b);
-    rows(0, pb);
+  if (binned)
+    hipLaunchKernelGGL(fine ? k_mpm_g2p_binned<kFineEdge> : k_mpm_g2p_binned<kCoarseEdge>, dim3(GP + kOobGroups),
+                       dim3(kBlock), 0, st, a, b);
+  rows(0, pb);
+  if (binned)
     hipLaunchKernelGGL(k_mpm_g2p_sums, dim3(pb), dim3(kBlock), 0, st, a);
-    hipLaunchKernelGGL((k_mpm_finish<21, FinNone>), dim3(1), dim3(kMpmFinishThreads), 0, st, (const double*)a.partials,
-                       pb, pb, a.totals + T_PDISP, FinNone{}, (uint64_t)0);
-  } else {
-    rows(0, pb);
+  else
     hipLaunchKernelGGL(k_mpm_g2p, dim3(pb), dim3(kBlock), 0, st, a);
-    hipLaunchKernelGGL((k_mpm_finish<21, FinNone>), dim3(1), dim3(kMpmFinishThreads), 0, st, (const double*)a.partials,
-                       pb, pb, a.totals + T_PDISP, FinNone{}, (uint64_t)0);
-  }
+  g2p_rows = next_table(pb, 21);
+  hipLaunchKernelGGL(k_mpm_finish_stages, dim3(3), dim3(kMpmFinishThreads), 0, st, p2g_rows, grid_rows, g2p_rows,
+                     a.totals);
   rows(0, pb);
   hipLaunchKernelGGL(k_mpm_radial, dim3(pb), dim3(kBlock), 0, st, a);
   hipLaunchKernelGGL((k_mpm_finish<3, FinMpmReport>), dim3(1), dim3(kMpmFinishThreads), 0, st,
-                     (const double*)a.partials, pb, pb, a.totals + T_RSUM, FinMpmReport{a.totals, a.report, a.dt},
+                     (const double*)table, pb, pb, a.totals + T_RSUM, FinMpmReport{a.totals, a.report, a.dt},
                      kRadialMax);
   HFSI_LAUNCH_CHECK();
   if (tile_path) {
