@@ -1272,6 +1272,14 @@ struct ReportArgs {
 constexpr int kReportSlots = 54;
 constexpr uint64_t kReportMaxMask = 0x9249249249249ull;  // bits 0, 3, 6, ..., 51
 
+// Workgroups (two per CU) up to 16 cells per lane; larger grids take more.  The pass is bound by its
+// reduction: 54 float64 slots over a wavefront are some 1300 instructions, as much as 20 cells per lane, so
+// fewer wavefronts with more cells each are faster.  With a workgroup per 256 cells (up to 2048) and one
+// finishing workgroup for all slots a report took 18.8 + 23.6 us at 64^3 and 33.2 + 40.8 us at 150 x 97 x
+// 118 cells; with 512 and a finishing workgroup per slot 13.3 + 3.8 and 24.8 + 4.4 us (256: 11.7 and 34.6 us
+// for the pass, 1024: 18.7 and 23.9 us).
+constexpr uint32_t kReportBlocks = 512;
+
 __global__ void __launch_bounds__(kBlock) k_div_report(ReportArgs a) {
   constexpr int NS = kReportSlots;
   __shared__ double lds[NS * (kBlock / 64)];
@@ -1335,6 +1343,25 @@ __global__ void __launch_bounds__(kBlock) k_div_report(ReportArgs a) {
   }
   // max for slot*3, sums otherwise
   block_partials<NS>(acc, a.partials, lds, kReportMaxMask);
+}
+
+// Combine the report's partial rows, a workgroup per slot (the rows come from every XCD: each load is a
+// round trip past this XCD's L2, and the slots' trips run side by side).
+__global__ void __launch_bounds__(kFinishThreads) k_finish_report(const double* partials, uint32_t nblocks,
+                                                                   double* totals) {
+  __shared__ double lds[kFinishThreads / 64];
+  const uint32_t s = blockIdx.x;
+  const bool mx = (kReportMaxMask >> s) & 1;
+  double acc[1] = {mx ? -INFINITY : 0.0};
+  for (uint32_t b = threadIdx.x; b < nblocks; b += kFinishThreads) {
+    const double p = partials[(size_t)b * kReportSlots + s];
+    acc[0] = mx ? fmax(acc[0], p) : acc[0] + p;
+  }
+  if (mx)
+    block_reduce<1>(acc, lds, 1ull);
+  else
+    block_reduce<1>(acc, lds, 0ull);
+  if (threadIdx.x == 0) totals[s] = acc[0];
 }
 
 // ---------------------------------------------------------------------------
@@ -4633,8 +4660,10 @@ int hfsi_fluid_divergence_report(hfsi_fluid* h, const float* divergence, const f
   a.partials = h->partials;
   a.counter = h->counter;
   a.totals = h->totals;
-  hipLaunchKernelGGL(k_div_report, dim3(blocks_for(a.g.n)), dim3(kBlock), 0, st, a);
-  finish_sums<kReportSlots>(h, blocks_for(a.g.n), FinNone{}, st, kReportMaxMask);
+  const uint32_t nb = std::min(blocks_for(a.g.n), std::max(kReportBlocks, blocks_for(a.g.n / 16)));
+  hipLaunchKernelGGL(k_div_report, dim3(nb), dim3(kBlock), 0, st, a);
+  hipLaunchKernelGGL(k_finish_report, dim3(kReportSlots), dim3(kFinishThreads), 0, st, (const double*)h->partials, nb,
+                     h->totals);
   HFSI_LAUNCH_CHECK();
   HFSI_CHECK(hipMemcpyAsync(h->host_totals, h->totals, 54 * sizeof(double), hipMemcpyDeviceToHost, st));
   HFSI_CHECK(hipStreamSynchronize(st));

@@ -128,6 +128,24 @@ def test_vcycle_ref64_matches_oracle(shape, graded, outlet):
     np.testing.assert_allclose(got, want, rtol=0, atol=1e-6 * np.abs(want).max())
 
 
+@pytest.mark.parametrize("outlet", [False, True])
+@pytest.mark.parametrize("shape", [(5, 4, 6), (9, 7, 33), (4, 67, 10), (70, 62, 58), (130, 34, 65)])
+def test_vcycle_edges_of_tail_and_restriction_tiles(shape, outlet):
+    """Levels of one to a few cells per axis in the single-workgroup tail, and fine levels whose coarse cells
+    fill no restriction tile; the tolerance of test_vcycle_ref64_matches_oracle."""
+    _say(f"vcycle edges shape={shape} outlet={outlet}")
+    w, obst = _graded(shape, 15), _obstacle(shape, 15, 0.05)
+    r = np.where(obst == 0, np.random.default_rng(16).normal(size=shape), 0.0)
+    s = _solver(w)
+    s.obstacle.from_numpy(obst)
+    s._set_masks()
+    rt = _t(r, torch.float64)
+    z = torch.zeros_like(rt)
+    _ok(s, s._lib.hfsi_fluid_vcycle(s._handle, rt.data_ptr(), z.data_ptr(), 1, 2, 24, 2, int(outlet), _stream()))
+    want = F.vcycle(r, F.build_hierarchy(w, obst), outlet)
+    np.testing.assert_allclose(z.cpu().numpy(), want, rtol=0, atol=1e-6 * np.abs(want).max())
+
+
 def _cg(s, div, precision, tol, max_it, outlet, remove_mean, precond=2, true_exit=0, check=16, true_res=0):
     from easyfsi_amd import _lib
 
@@ -331,6 +349,34 @@ def test_report_matches_oracle_stats():
         got = s.divergence_residual_stats(interior_only=interior)
         want = F.divergence_l2_stats(div, src, obst, interior, residual=True)
         assert got["l2"] == pytest.approx(want["l2"], rel=1e-12)
+
+
+@pytest.mark.parametrize("shape", [(4, 4, 4), (64, 64, 33), (90, 97, 118), (150, 117, 130)])
+def test_report_at_the_edges_of_its_grid(shape):
+    """One workgroup; just over one cell per lane of 512 workgroups; several cells per lane; more than 512
+    workgroups.  Maxima and counts are exact; the sums of squares, all terms positive and float64, differ by
+    at most n 2^-53 < 3e-10 relative from NumPy's in another order."""
+    rng = np.random.default_rng(41)
+    obst = _obstacle(shape, 41)
+    div = rng.normal(size=shape).astype(np.float32)
+    src = (rng.normal(size=shape) * 0.1).astype(np.float32)
+    s = _solver(_graded(shape, 41))
+    for field, value in ((s.obstacle, obst), (s.divergence, div), (s.volume_source_s, src)):
+        field.from_numpy(value)
+    s._set_masks()
+    got = s._report_slots()
+    free = obst == 0
+    inner = np.zeros(shape, bool)
+    inner[1:-1, 1:-1, 1:-1] = True
+    raw = np.abs(div.astype(np.float64))
+    res = np.abs(div.astype(np.float64) - src.astype(np.float64))
+    for slot, v, m in ((0, raw, free), (1, res, free), (2, raw, free & inner), (3, res, free & inner),
+                       (6, raw, free), (7, res, free)):
+        assert got[slot, 2] == m.sum()
+        assert got[slot, 0] == (v[m].max() if m.any() else 0.0)
+        assert got[slot, 1] == pytest.approx(float((v[m] ** 2).sum()), rel=3e-10)
+    assert got[8, 2] + got[10, 2] == free.sum() and got[4, 2] == 0
+    assert got[8, 1] + got[10, 1] == pytest.approx(got[0, 1], rel=3e-10)
 
 
 @pytest.mark.parametrize("seed", [0, 1])
