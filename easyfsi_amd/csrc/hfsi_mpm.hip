@@ -8,11 +8,11 @@
 //   k_mpm_g2p        27-node gather, APIC C, x += dt v, F <- (I + dt C) F,
 //                    surface normal / area update
 //   k_mpm_radial     centroid-relative radial stretch diagnostics
-// Binned path (default): particles binned by 8^3-node block; P2G as a per-particle
+// Binned path (default): particles binned by block of 4^3 or 8^3 nodes; P2G as a per-particle
 // pass (k_mpm_p2g_prepare, k_mpm_p2g_prepare_svd) and a per-cell scatter into
-// LDS tiles (k_mpm_p2g_cells, k_mpm_p2g_force); the grid update gathers the tiles
-// (k_mpm_grid_gather); G2P from an LDS velocity tile per block (k_mpm_g2p_binned,
-// k_mpm_g2p_oob) with its report sums in a pass of their own (k_mpm_g2p_sums).
+// LDS tiles (k_mpm_p2g_fine or k_mpm_p2g_cells, k_mpm_p2g_force); the grid update gathers the tiles
+// (k_mpm_grid_gather); G2P from an LDS velocity tile per block (k_mpm_g2p_binned)
+// with its report sums in a pass of their own (k_mpm_g2p_sums).
 // The report quantities are reduced deterministically (workgroup partials,
 // combined in workgroup order by a one-workgroup finish launch); the final
 // 34-value report snapshot is assembled on the device.

@@ -136,7 +136,7 @@ class NeoHookeanMpmState:
             self._handle = None
 
     def set_p2g_mode(self, mode: str) -> None:
-        """'binned' (default): particles bucketed by 8^3-node block, accumulated in LDS; 'atomic': every
+        """'binned' (default): particles bucketed by block of 4^3 or 8^3 nodes, accumulated in LDS; 'atomic': every
         particle scatters its 27 node contributions with global atomics."""
         modes = {"binned": 0, "atomic": 1}
         if mode not in modes:

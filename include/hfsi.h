@@ -314,10 +314,10 @@ int hfsi_mpm_create(hfsi_mpm** out, int32_t particle_capacity, const double* bou
                     const int32_t* grid_nodes3, void* stream);
 int hfsi_mpm_destroy(hfsi_mpm* h);
 
-/* P2G scatter: HFSI_MPM_P2G_BINNED (default) buckets particles by 8^3-node
- * block and accumulates each block in an LDS tile; the tiles are stored
+/* P2G scatter: HFSI_MPM_P2G_BINNED (default) buckets particles by block of
+ * 4^3 nodes (states of up to 2^19 particles) or 8^3 nodes and accumulates each block in an LDS tile; the tiles are stored
  * whole and the grid update sums, for every node, the (up to 8) tiles that
- * cover it in a fixed order (grids of more than 65536 blocks add each tile
+ * cover it in a fixed order (grids of more than 65536 blocks of 8^3 nodes add each tile
  * to the grid with global atomics instead).  HFSI_MPM_P2G_ATOMIC scatters
  * every particle's 27 node contributions with global float atomics.  Same
  * arithmetic per particle; float summation order differs. */
